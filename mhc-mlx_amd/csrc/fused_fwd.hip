@@ -16,6 +16,7 @@
 
 #include "mhc_device.hpp"
 #include "mhc_generic.hpp"
+#include "mhc_lf32.hpp"
 #include "mhc_mfma32.hpp"
 #include "mhc_host.hpp"
 #include "mhc_plan.hpp"
@@ -584,6 +585,13 @@ __global__ __launch_bounds__(SPW == 2 ? 512 : 1024) void fused_fwd_mfma16_kernel
 
 namespace {
 
+GenArgs gen_args(const FwdArgs& A) {
+  GenArgs G{};
+  G.x = A.x; G.out = A.out; G.M = A.M; G.hpre = A.hpre; G.hpost = A.hpost; G.w = A.w; G.inv_rms = A.inv_rms;
+  G.T = A.T; G.M_ts = A.M_ts; G.h_ts = A.h_ts; G.n = A.n; G.C = A.C; G.h_mode = A.h_mode; G.eps = A.eps;
+  return G;
+}
+
 // MFMA kernel for n == 16 with 16-bit x.  Returns 1 when the shape is not
 // covered (the caller then uses fused_fwd_kernel).
 template <typename XT, typename OT, bool PT>
@@ -671,7 +679,9 @@ int launch_fwd(FwdArgs A, hipStream_t stream) {
     if (rc != 1) return rc;
   }
   if constexpr (NMAX == 16) {
-    const int rc = launch_fwd_mfma16<XT, OT, PT>(A, stream);
+    int rc = launch_fwd_mfma16<XT, OT, PT>(A, stream);
+    if (rc != 1) return rc;
+    rc = lf32_fused_fwd(gen_args(A), dtype_code<XT>(), dtype_code<OT>(), stream);
     if (rc != 1) return rc;
   }
   A.nchunks = (int)ceil_div(A.C, V);
@@ -751,12 +761,11 @@ extern "C" int mhc_fused_fwd(const void* x, int x_dtype, const float* M, int64_t
     Mf32Args F{};
     F.x = x; F.out = out; F.inv_rms = inv_rms; F.M = M; F.hpre = h_pre; F.hpost = h_post; F.w = rms_weight;
     F.T = T; F.M_ts = M_token_stride; F.h_ts = h_token_stride; F.n = n; F.C = C; F.h_mode = h_mode; F.eps = eps;
-    const int rc = mf32_fused_fwd(F, x_dtype, out_dtype, (hipStream_t)stream);
+    int rc = mf32_fused_fwd(F, x_dtype, out_dtype, (hipStream_t)stream);
     if (rc != 1) return rc;
-    GenArgs G{};
-    G.x = x; G.out = out; G.M = M; G.hpre = h_pre; G.hpost = h_post; G.w = rms_weight;
-    G.inv_rms = inv_rms; G.T = T; G.M_ts = M_token_stride; G.h_ts = h_token_stride; G.n = n;
-    G.C = C; G.h_mode = h_mode; G.eps = eps;
+    const GenArgs G = gen_args(A);
+    rc = lf32_fused_fwd(G, x_dtype, out_dtype, (hipStream_t)stream);
+    if (rc != 1) return rc;
     return gen_fused_fwd(G, x_dtype, out_dtype, (hipStream_t)stream);
   }
   const int V = fwd_vec_width(nmax_for(n));

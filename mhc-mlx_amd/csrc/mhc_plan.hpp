@@ -7,6 +7,7 @@
 #include <stdlib.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "mhc_host.hpp"
 
@@ -35,6 +36,11 @@ inline int dtype_bytes(int code) {
     case MHC_DTYPE_F16: return 2;
     default: return 0;
   }
+}
+
+template <typename T>
+constexpr int dtype_code() {
+  return sizeof(T) == 4 ? MHC_DTYPE_F32 : (std::is_same<T, __bf16>::value ? MHC_DTYPE_BF16 : MHC_DTYPE_F16);
 }
 
 struct ThreadPlan {

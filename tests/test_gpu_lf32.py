@@ -1,0 +1,77 @@
+"""GPU parity of the fp32-MFMA layer forward (csrc/lf32_fwd.hip) against the float64 oracle.
+
+It serves 8 < n <= 64 where the 16-bit MFMA kernels do not: fp32 or mixed dtypes, any C and row alignment.  The
+sizes sit at the edges of its splits: the 16-row blocks of streams (n = 9, 16, 17, 32, 33, 48, 49, 64), the
+64-channel slabs (C below, at and past a multiple), the element-wise rows (C not a multiple of 4), one slab per wave,
+two and four, and the two-pass form for longer tokens.
+"""
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import mhc_oracle as O
+from tests._helpers import TOL, dev_tensor, np_of, params, rel_err, rng, to_dtype_np
+
+from mhc_mlx_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+EPS = 1e-5
+SHAPES = [(3, 9, 4), (70, 16, 64), (5, 16, 68), (300, 12, 100), (7, 16, 516), (4, 13, 1100), (3, 16, 2304),
+          (40, 17, 65), (9, 32, 512), (6, 32, 516), (3, 24, 1030), (5, 32, 1096), (2, 20, 2500),
+          (4, 33, 61), (6, 48, 512), (3, 49, 130), (5, 64, 192), (2, 64, 1000), (2, 40, 516)]
+
+
+def _inputs(T, n, C, xdt, gdt, per_token):
+    g = rng(9100 + T + n + C)
+    x = to_dtype_np(g.standard_normal((T, n, C)), xdt)
+    dout = to_dtype_np(g.standard_normal((T, n, C)), gdt)
+    return x, dout, params(g, n, C, per_token_B=T if per_token else None)
+
+
+@pytest.mark.parametrize("T,n,C", SHAPES)
+@pytest.mark.parametrize("xdt,odt", [("f32", "f32"), ("bf16", "f32"), ("f16", "f16")])
+@pytest.mark.parametrize("per_token", [False, True])
+def test_lf32_forward(T, n, C, xdt, odt, per_token, knobs):
+    """Every split, with one workgroup per CU and with several tokens per workgroup; the fp32 results differ in their
+    last bits from the VALU kernels' (MHC_FWD_MFMA=0), so the MFMA kernel ran."""
+    x, _, ps = _inputs(T, n, C, xdt, xdt, per_token)
+    xt, pt = dev_tensor(x, xdt), [dev_tensor(v) for v in ps]
+    fn = ops.mhc_layer_forward_dynamic if per_token else ops.mhc_layer_forward
+
+    def run():
+        with torch.no_grad():
+            return fn(xt, *pt, sinkhorn_iters=20, eps=EPS, output_dtype=None if odt == "f32" else xt.dtype)
+
+    out, again = run(), run()
+    assert torch.equal(out, again)
+    ref = O.mhc_forward_reference(x, *ps, sinkhorn_iters=20, eps=EPS)
+    # fp32: 64 products of rounded fp32 factors, summed in fp32; 16-bit: one rounding of that
+    tol = 1e-5 if odt == "f32" else TOL[odt]
+    assert rel_err(np_of(out), ref) < tol, rel_err(np_of(out), ref)
+    knobs("MHC_FWD_MFMA", 0)
+    assert rel_err(np_of(run()), np_of(out)) < tol
+    if odt == "f32" and T * n * C > 20000:
+        assert not torch.equal(run(), out)
+
+
+def test_lf32_forward_unaligned_and_non_finite():
+    """x and out at addresses that are no multiple of a row's four elements take the element-wise rows, with the same
+    values; an infinity and a NaN stay in the tokens and channels that they belong to."""
+    T, n, C = 6, 20, 256
+    x, _, ps = _inputs(T, n, C, "f32", "f32", False)
+    pt = [dev_tensor(v) for v in ps]
+    x[1, 3, 70] = np.inf
+    x[4, 19, 255] = np.nan
+    buf = torch.empty(T * n * C + 1, device="cuda")
+    off = buf[1:].view(T, n, C)
+    off.copy_(dev_tensor(x))
+    with torch.no_grad():
+        a = ops.mhc_layer_forward(dev_tensor(x), *pt, eps=EPS)
+        b = ops.mhc_layer_forward(off, *pt, eps=EPS)
+    assert torch.equal(torch.nan_to_num(a, 7.0), torch.nan_to_num(b, 7.0))
+    bad = ~torch.isfinite(a)
+    assert not bad[[0, 2, 3, 5]].any()
+    assert bad[1, :, 70].all() and bad[4].all()  # a NaN reaches its token's RMS factor
+    assert torch.isfinite(a[1][:, [0, 69, 71, 255]]).all()
