@@ -21,6 +21,7 @@
 
 #include "mhc_device.hpp"
 #include "mhc_generic.hpp"
+#include "mhc_lf32.hpp"
 #include "mhc_mfma32.hpp"
 #include "mhc_host.hpp"
 #include "mhc_plan.hpp"
@@ -1488,6 +1489,14 @@ void set_rows(BwdArgs& A, const BwdLayout& L) {
   A.P = L.P;
 }
 
+GenArgs gen_args(const BwdArgs& A, const BwdLayout& L) {
+  GenArgs G{};
+  G.x = A.x; G.g = A.g; G.out = A.dx; G.M = A.M; G.hpre = A.hpre; G.hpost = A.hpost; G.w = A.w; G.part = A.part;
+  G.dM_tok = A.dM_tok; G.dpre_tok = A.dpre_tok; G.dpost_tok = A.dpost_tok; G.T = A.T; G.M_ts = A.M_ts;
+  G.h_ts = A.h_ts; G.n = A.n; G.C = A.C; G.Cp = L.Cp; G.P = L.P; G.h_mode = A.h_mode; G.eps = A.eps;
+  return G;
+}
+
 // Layer-wide n <= 8 (fused_bwd_lw_kernel).  Returns 1 when the shape is not
 // covered (C too large for one chunk per thread), so the caller falls back
 // to fused_bwd_kernel.
@@ -1656,6 +1665,10 @@ int launch_bwd(BwdArgs A, const BwdLayout& L, int64_t* num_partials, hipStream_t
       if (rc != 1) return rc;
     }
   }
+  if constexpr (NMAX == 16) {
+    const int rc = lf32_fused_bwd(gen_args(A, L), dtype_code<XT>(), dtype_code<GT>(), L.gmax, stream, num_partials);
+    if (rc != 1) return rc;
+  }
   return launch_bwd_tile<NMAX, XT, GT, PT>(A, L, num_partials, stream);
 }
 
@@ -1737,15 +1750,12 @@ extern "C" int mhc_fused_bwd_partials(const void* x, int x_dtype, const void* do
     F.part = (float*)workspace; F.T = T; F.M_ts = M_token_stride; F.h_ts = h_token_stride; F.n = n; F.C = C;
     F.Cp = L.Cp; F.P = L.P; F.h_mode = h_mode; F.eps = eps;
     F.dM_tok = dM_tok; F.dpre_tok = dh_pre_tok; F.dpost_tok = dh_post_tok;
-    const int rc = mf32_fused_bwd(F, x_dtype, dout_dtype, L.gmax, (hipStream_t)stream, num_partials);
+    int rc = mf32_fused_bwd(F, x_dtype, dout_dtype, L.gmax, (hipStream_t)stream, num_partials);
     if (rc != 1) return rc;
-    GenArgs G{};
-    G.x = x; G.g = dout; G.out = dx; G.M = M; G.hpre = h_pre; G.hpost = h_post; G.w = rms_weight;
-    G.part = (float*)workspace;
+    GenArgs G = gen_args(A, L);
+    rc = lf32_fused_bwd(G, x_dtype, dout_dtype, L.gmax, (hipStream_t)stream, num_partials);
+    if (rc != 1) return rc;
     G.scratch = (float*)((char*)workspace + L.scratch_off);
-    G.dM_tok = dM_tok; G.dpre_tok = dh_pre_tok; G.dpost_tok = dh_post_tok;
-    G.T = T; G.M_ts = M_token_stride; G.h_ts = h_token_stride; G.n = n; G.C = C; G.Cp = L.Cp;
-    G.P = L.P; G.h_mode = h_mode; G.eps = eps;
     return gen_fused_bwd(G, x_dtype, dout_dtype, (hipStream_t)stream, num_partials);
   }
   const int V = bwd_vec_width(nmax_for(n));

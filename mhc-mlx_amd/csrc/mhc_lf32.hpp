@@ -1,6 +1,6 @@
-// The layer's forward on fp32 MFMA for every 8 < n <= 64 shape that the 16-bit MFMA
+// The layer on fp32 MFMA for every 8 < n <= 64 shape that the 16-bit MFMA
 // kernels do not take: fp32 or mixed dtypes, channel counts that are no
-// multiple of 128, unaligned rows (lf32_fwd.hip).
+// multiple of 128, unaligned rows (lf32_fwd.hip, lf32_bwd.hip).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -14,6 +14,16 @@ namespace mhc {
 // out = M x + p * rms_norm(a^T x) w; layer-wide or per-token parameters.
 // Returns 1 when the shape is not covered.
 int lf32_fused_fwd(const GenArgs& A, int x_dtype, int out_dtype, hipStream_t s);
+
+// Partial-sums pass of the VJP: dx, and one partial row per workgroup
+// [dw C | pad | dM n*n | dA n | dP n] (at most gmax workgroups); per token
+// parameters: the token's dM, dh_pre and dh_post, and [dw C | pad] rows.
+// Returns 1 when the shape is not covered.
+int lf32_fused_bwd(const GenArgs& A, int x_dtype, int g_dtype, int64_t gmax, hipStream_t s, int64_t* num_partials);
+
+// lf32_fused_bwd for one dtype of x (one source file each: the kernels compile in parallel).
+int lf_bwd_bf16(const GenArgs& A, bool g_f32, int64_t gmax, hipStream_t s, int64_t* num_partials);
+int lf_bwd_f16(const GenArgs& A, bool g_f32, int64_t gmax, hipStream_t s, int64_t* num_partials);
 
 constexpr int kLfSlab = 64;       // channels per slab: four per lane of a 16-lane group
 constexpr int kLfMaxWaves = 8;    // waves per workgroup

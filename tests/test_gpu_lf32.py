@@ -1,7 +1,7 @@
-"""GPU parity of the fp32-MFMA layer forward (csrc/lf32_fwd.hip) against the float64 oracle.
+"""GPU parity of the fp32-MFMA layer kernels (csrc/lf32_fwd.hip, csrc/lf32_bwd.hip) against the float64 oracle.
 
-It serves 8 < n <= 64 where the 16-bit MFMA kernels do not: fp32 or mixed dtypes, any C and row alignment.  The
-sizes sit at the edges of its splits: the 16-row blocks of streams (n = 9, 16, 17, 32, 33, 48, 49, 64), the
+They serve 8 < n <= 64 where the 16-bit MFMA kernels do not: fp32 or mixed dtypes, any C and row alignment.  The
+sizes sit at the edges of their splits: the 16-row blocks of streams (n = 9, 16, 17, 32, 33, 48, 49, 64), the
 64-channel slabs (C below, at and past a multiple), the element-wise rows (C not a multiple of 4), one slab per wave,
 two and four, and the two-pass form for longer tokens.
 """
@@ -11,7 +11,7 @@ import pytest
 import torch
 
 from oracle import mhc_oracle as O
-from tests._helpers import TOL, dev_tensor, np_of, params, rel_err, rng, to_dtype_np
+from tests._helpers import GRAD_TOL, TOL, dev_tensor, np_of, params, rel_err, rng, to_dtype_np
 
 from mhc_mlx_amd import ops
 
@@ -75,3 +75,57 @@ def test_lf32_forward_unaligned_and_non_finite():
     assert not bad[[0, 2, 3, 5]].any()
     assert bad[1, :, 70].all() and bad[4].all()  # a NaN reaches its token's RMS factor
     assert torch.isfinite(a[1][:, [0, 69, 71, 255]]).all()
+
+
+@pytest.mark.parametrize("T,n,C", SHAPES)
+@pytest.mark.parametrize("xdt,gdt", [("f32", "f32"), ("bf16", "f32"), ("f16", "f16")])
+@pytest.mark.parametrize("per_token", [False, True])
+@pytest.mark.parametrize("grid", [None, 2])
+def test_lf32_backward(T, n, C, xdt, gdt, per_token, grid, knobs):
+    """Every gradient, with a grid of the whole chip and with two workgroups that walk many tokens each; reruns are
+    bitwise equal, and fp32 results differ in their last bits from the VALU kernels' (MHC_BWD_MFMA=0)."""
+    if grid is not None:
+        knobs("MHC_BWD_GRID", grid)
+    x, dout, ps = _inputs(T, n, C, xdt, gdt, per_token)
+    fn = ops.mhc_layer_forward_dynamic if per_token else ops.mhc_layer_forward
+
+    def run():
+        xt = dev_tensor(x, xdt).requires_grad_(True)
+        pt = [dev_tensor(v).requires_grad_(True) for v in ps]
+        out = fn(xt, *pt, sinkhorn_iters=20, eps=EPS, output_dtype=None if gdt == "f32" else xt.dtype)
+        return torch.autograd.grad(out, [xt, *pt], dev_tensor(dout, gdt))
+
+    got, again = run(), run()
+    for a, b in zip(got, again):
+        assert torch.equal(a, b)
+    refs = O.mhc_backward_reference(x, *ps, dout, sinkhorn_iters=20, eps=EPS)
+    names = ("dx", "dH_pre", "dH_post", "dH_res", "d_w")
+    for name, a, r in zip(names, got, refs):
+        tol = TOL[xdt] if name == "dx" else GRAD_TOL
+        assert rel_err(np_of(a), r) < tol, (name, rel_err(np_of(a), r))
+    if grid is None and T * n * C > 20000:
+        knobs("MHC_BWD_MFMA", 0)
+        valu = run()
+        assert not all(torch.equal(a, b) for a, b in zip(got[1:], valu[1:]))
+
+
+@pytest.mark.parametrize("n,C", [(12, 100), (24, 260), (40, 68)])
+def test_lf32_backward_activated_h(n, C):
+    """The op-level VJP (activated H in and out) takes the same kernels."""
+    T = 9
+    x, dout, (hpre, hpost, hres, w) = _inputs(T, n, C, "f32", "f32", False)
+    M = O.mixing_matrix_from_logits(hres, 20, EPS)
+    a, p = 1.0 / (1.0 + np.exp(-hpre)), 2.0 / (1.0 + np.exp(-hpost))
+    xt = dev_tensor(x).requires_grad_(True)
+    ts = [dev_tensor(v).requires_grad_(True) for v in (a, p)]
+    Mt = dev_tensor(M).requires_grad_(True)
+    wt = dev_tensor(w).requires_grad_(True)
+    out = ops.mhc_forward_fused_hip_autograd(xt, Mt, ts[0], ts[1], wt, eps=EPS)
+    got = torch.autograd.grad(out, [xt, Mt, ts[0], ts[1], wt], dev_tensor(dout))
+    ref_in = [t.detach().double().requires_grad_(True) for t in (xt, Mt, ts[0], ts[1], wt)]
+    xd, Md, ad, pd, wd = ref_in
+    y = (ad[None, :, None] * xd).sum(1)
+    yn = y * torch.rsqrt(y.square().mean(-1, keepdim=True) + EPS) * wd
+    ref = torch.matmul(Md, xd) + pd[None, :, None] * yn[:, None, :]
+    for g, r in zip(got, torch.autograd.grad(ref, ref_in, dev_tensor(dout).double())):
+        assert rel_err(np_of(g), r.cpu().numpy()) < GRAD_TOL
