@@ -204,37 +204,55 @@ __global__ __launch_bounds__(PT ? 64 : (NB > 2 ? 256 : 64 * kLfMaxWaves)) void l
     }
     issue_fence();
   };
-  // dM and the dot products over the slab in LDS
+  // dM and the dot products over the slab in LDS.  The slab's products are summed by themselves first: one chain over all
+  // of a wave's slabs would round every product against the whole sum (dH_res at 30000 x 9 x 400 bf16 1.8e-6 off the
+  // exact sum instead of 0.3e-6).  At n > 48 the row blocks of g go in two passes (four per token), so that these partial sums fit.
+  constexpr int IB = NB > 3 ? (PT ? 1 : 2) : NB;
   auto sums = [&] {
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      __builtin_amdgcn_sched_barrier(0);  // the four steps' operands at once would take 80-112 registers
-      const int c = 16 * k + 4 * q;
-      f32x4 gv[NB], xv[NB];
+    for (int I0 = 0; I0 < NB; I0 += IB) {
+      f32x4 part[IB][NB];
 #pragma unroll
-      for (int I = 0; I < NB; ++I) {
-        gv[I] = *reinterpret_cast<const f32x4*>(sg + (16 * I + r) * kLfPitch + c);
-        xv[I] = *reinterpret_cast<const f32x4*>(sx + (16 * I + r) * kLfPitch + c);
-      }
-      const f32x4 yv = *reinterpret_cast<const f32x4*>(sc + c);
-      const f32x4 dw = *reinterpret_cast<const f32x4*>(sc + kLfSlab + c);
-      const f32x4 yw = *reinterpret_cast<const f32x4*>(sc + 2 * kLfSlab + c);
+      for (int I = 0; I < IB; ++I)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
+        for (int J = 0; J < NB; ++J) part[I][J] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int I = 0; I < NB; ++I)
+      for (int k = 0; k < 4; ++k) {
+        __builtin_amdgcn_sched_barrier(0);  // the four steps' operands at once would take 80-112 registers
+        const int c = 16 * k + 4 * q;
+        f32x4 gv[IB], xv[NB];
 #pragma unroll
-          for (int J = 0; J < NB; ++J) dm[I][J] = lf_mfma(gv[I][e], xv[J][e], dm[I][J]);
+        for (int I = 0; I < IB; ++I)
+          gv[I] = *reinterpret_cast<const f32x4*>(sg + (16 * (I0 + I) + r) * kLfPitch + c);
 #pragma unroll
-        for (int I = 0; I < NB; ++I) {
-          ux[I] = fmaf(xv[I][e], dw[e], ux[I]);
-          vx[I] = fmaf(xv[I][e], yv[e], vx[I]);
-          ug[I] = fmaf(gv[I][e], yw[e], ug[I]);
+        for (int J = 0; J < NB; ++J) xv[J] = *reinterpret_cast<const f32x4*>(sx + (16 * J + r) * kLfPitch + c);
+        const f32x4 yv = *reinterpret_cast<const f32x4*>(sc + c);
+        const f32x4 dw = *reinterpret_cast<const f32x4*>(sc + kLfSlab + c);
+        const f32x4 yw = *reinterpret_cast<const f32x4*>(sc + 2 * kLfSlab + c);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+#pragma unroll
+          for (int I = 0; I < IB; ++I)
+#pragma unroll
+            for (int J = 0; J < NB; ++J) part[I][J] = lf_mfma(gv[I][e], xv[J][e], part[I][J]);
+#pragma unroll
+          for (int I = 0; I < IB; ++I) ug[I0 + I] = fmaf(gv[I][e], yw[e], ug[I0 + I]);
+          if (I0 == 0) {
+#pragma unroll
+            for (int J = 0; J < NB; ++J) {
+              ux[J] = fmaf(xv[J][e], dw[e], ux[J]);
+              vx[J] = fmaf(xv[J][e], yv[e], vx[J]);
+            }
+          }
         }
-      }
-      // the dot products stay here: moved to their use after the barrier they would hold every operand until then
+        // the dot products stay here: moved to their use after the barrier they would hold every operand until then
 #pragma unroll
-      for (int I = 0; I < NB; ++I) asm volatile("" : "+v"(ux[I]), "+v"(vx[I]), "+v"(ug[I]));
+        for (int I = 0; I < NB; ++I) asm volatile("" : "+v"(ux[I]), "+v"(vx[I]), "+v"(ug[I]));
+      }
+#pragma unroll
+      for (int I = 0; I < IB; ++I)
+#pragma unroll
+        for (int J = 0; J < NB; ++J) dm[I0 + I][J] += part[I][J];
     }
   };
   // M^T g of g[j] (n <= 32)
