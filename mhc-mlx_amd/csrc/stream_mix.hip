@@ -13,6 +13,7 @@
 #include "mhc_generic.hpp"
 #include "mhc_host.hpp"
 #include "mhc_mix32.hpp"
+#include "mhc_mxf32.hpp"
 #include "mhc_plan.hpp"
 #include "mhc_reduce.hpp"
 
@@ -829,6 +830,12 @@ int by_dtype(int code, F&& f) {
   }
 }
 
+// Whether the post-combine's MFMA kernels are asked first (they may decline).  They pad n to 16 rows: at n <= 4, and at
+// n <= 8 with whole aligned chunks, mix_add_*_kernel streams as fast or faster (8192 x 3 x 341 fp32 forward 33 against
+// 38 us); with ragged rows at n > 4 and everywhere above n = 8 the VALU kernel is the slower one (VJP call 8192 x 6 x 170
+// bf16 98 against 47 us, 8192 x 12 x 128 bf16 66 against 34 us).
+bool mxf_takes(int n, bool vec) { return n > 8 || (n > 4 && !vec); }
+
 int mix_rows(int n) { return round_up(n * n + n, 4); }
 
 }  // namespace
@@ -861,12 +868,16 @@ extern "C" int mhc_stream_mix_add_fwd(const void* x, int x_dtype, const void* y,
   const int64_t blocks = mix_grid(T * A.nchunks, device_cu_count(), kKnobMixFwdGrid, 8);
   hipStream_t s = (hipStream_t)stream;
   const int ydt = y ? y_dtype : x_dtype;
-  if (nmax_for(n) == 0) {
-    Mix32Args F{};
-    F.x = x; F.y = y; F.out = out; F.M = M; F.hpre = h_pre; F.hpost = h_post; F.T = T; F.n = n; F.C = C;
-    F.h_mode = h_mode;
-    const int rc = mix32_fwd(F, x_dtype, ydt, out_dtype, s);
+  Mix32Args F{};
+  F.x = x; F.y = y; F.out = out; F.M = M; F.hpre = h_pre; F.hpost = h_post; F.T = T; F.n = n; F.C = C;
+  F.h_mode = h_mode;
+  if (mxf_takes(n, A.vec)) {
+    int rc = mix32_fwd(F, x_dtype, ydt, out_dtype, s);
     if (rc != 1) return rc;
+    rc = mxf_fwd(F, x_dtype, ydt, out_dtype, s);
+    if (rc != 1) return rc;
+  }
+  if (nmax_for(n) == 0) {
     GenArgs G{};
     G.x = x; G.y = y; G.out = out; G.M = M; G.hpre = h_pre; G.hpost = h_post; G.T = T; G.n = n;
     G.C = C; G.h_mode = h_mode;
@@ -935,22 +946,23 @@ extern "C" int mhc_stream_mix_add_bwd(const void* x, int x_dtype, const void* y,
   A.vec = io_vec_ok(C, V, {{x, dtype_bytes(x_dtype)}, {y, dtype_bytes(ydt)},
                            {dout, dtype_bytes(dout_dtype)}, {dy, dtype_bytes(ydt)}});
   hipStream_t s = (hipStream_t)stream;
-  int rc;
-  int64_t rows = G;  // partial rows written (the MFMA kernel may write fewer)
-  if (nmax_for(n) == 0) {
+  int rc = 1;
+  int64_t rows = G;  // partial rows written (the MFMA kernels choose their own count)
+  if (mxf_takes(n, A.vec)) {
     Mix32Args F{};
     F.x = x; F.y = y; F.g = dout; F.out = dx; F.dy = dy; F.M = M; F.hpre = h_pre; F.hpost = h_post;
     F.part = (float*)workspace; F.T = T; F.n = n; F.C = C; F.h_mode = h_mode; F.P = P;
     rc = mix32_bwd(F, x_dtype, ydt, dout_dtype, G, s, &rows);
-    if (rc == 1) {
-      GenArgs Gg{};
-      Gg.x = x; Gg.y = y; Gg.g = dout; Gg.out = dx; Gg.dy = dy; Gg.M = M; Gg.hpre = h_pre;
-      Gg.hpost = h_post; Gg.part = (float*)workspace; Gg.T = T; Gg.n = n; Gg.C = C; Gg.P = P;
-      Gg.h_mode = h_mode;
-      rows = G;
-      rc = gen_mix_bwd(Gg, x_dtype, ydt, dout_dtype, s, G);
-    }
-  } else rc = by_nmax(n, [&](auto nm) {
+    // (the caller's workspace may hold more rows than this call's widest items need)
+    if (rc == 1) rc = mxf_bwd(F, x_dtype, ydt, dout_dtype, (int64_t)(workspace_bytes / (P * sizeof(float))) - kMixSplit, s, &rows);
+  }
+  if (rc == 1 && nmax_for(n) == 0) {
+    GenArgs Gg{};
+    Gg.x = x; Gg.y = y; Gg.g = dout; Gg.out = dx; Gg.dy = dy; Gg.M = M; Gg.hpre = h_pre;
+    Gg.hpost = h_post; Gg.part = (float*)workspace; Gg.T = T; Gg.n = n; Gg.C = C; Gg.P = P;
+    Gg.h_mode = h_mode;
+    rc = gen_mix_bwd(Gg, x_dtype, ydt, dout_dtype, s, G);
+  } else if (rc == 1) rc = by_nmax(n, [&](auto nm) {
     constexpr int NM = decltype(nm)::value;
     return by_dtype(x_dtype, [&](auto* xp) {
       using XT = std::remove_pointer_t<decltype(xp)>;
@@ -975,7 +987,7 @@ extern "C" int mhc_stream_mix_add_bwd(const void* x, int x_dtype, const void* y,
     });
   });
   if (rc != MHC_OK) return rc;
-  float* part2 = (float*)workspace + (size_t)G * P;
+  float* part2 = (float*)workspace + (size_t)std::max(G, rows) * P;
   // about 64 rows per split: the split sums run in parallel workgroups, and
   // mix_final_kernel (one workgroup) then adds few rows per column
   const int S = (int)std::min<int64_t>(kMixSplit, ceil_div(rows, 64));

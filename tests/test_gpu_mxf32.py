@@ -1,0 +1,89 @@
+"""GPU parity of the fp32-MFMA post-combine (csrc/mxf32.hpp) against the float64 oracle.
+
+It serves MHCRewire's post-combine above n = 8 (and ragged rows above n = 4) where C is no multiple of 64.  The sizes
+sit at the edges of its splits: the 16-row blocks of streams, slabs of 64 columns that hold part of a token, one token
+or many, a partial last slab, rows taken one element at a time, and waves that walk several slabs.
+"""
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import mhc_oracle as O
+from tests._helpers import GRAD_TOL, TOL, dev_tensor, np_of, params, rel_err, rng, to_dtype_np
+
+from mhc_mlx_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(3, 5, 3), (70, 6, 18), (5, 8, 31), (40, 9, 4), (9, 16, 64), (33, 16, 20), (2, 13, 1000), (11, 17, 32),
+          (65, 32, 32), (7, 32, 2), (3, 24, 100), (5, 33, 12), (2, 48, 76), (9, 49, 7), (4, 64, 32), (1, 64, 1)]
+
+
+@pytest.mark.parametrize("T,n,C", SHAPES)
+@pytest.mark.parametrize("xdt,odt", [("f32", "f32"), ("bf16", "f32"), ("f16", "f16")])
+@pytest.mark.parametrize("grid", [None, 1])
+def test_mxf32_post_combine(T, n, C, xdt, odt, grid, knobs):
+    """Output and every gradient, reruns bitwise equal; with one workgroup per CU at most."""
+    if grid is not None:
+        knobs("MHC_MIX_FWD_GRID", grid)
+        knobs("MHC_MIX_BWD_GRID", grid)
+    g = rng(9300 + T + n + C)
+    x, y = (to_dtype_np(g.standard_normal((T, n, C)), xdt) for _ in range(2))
+    dout = to_dtype_np(g.standard_normal((T, n, C)), odt)
+    hpre, hpost, hres, _ = params(g, n, C)
+
+    def run():
+        ts = [dev_tensor(v, xdt).requires_grad_(True) for v in (x, y)]
+        ps = [dev_tensor(v).requires_grad_(True) for v in (hpre, hpost, hres)]
+        out = ops.post_combine(*ts, *ps, sinkhorn_iters=20, eps=1e-5, output_dtype=None if odt == "f32" else ts[0].dtype)
+        return [out.detach(), *torch.autograd.grad(out, [*ts, *ps], dev_tensor(dout, odt))]
+
+    got, again = run(), run()
+    for a, b in zip(got, again):
+        assert torch.equal(a, b)
+    refs = [O.post_combine(x, y, hpre, hpost, hres, 20, 1e-5),
+            *O.post_combine_backward(x, y, hpre, hpost, hres, dout, 20, 1e-5)]
+    for name, a, r in zip(("out", "dx", "dy", "dH_pre", "dH_post", "dH_res"), got, refs):
+        tol = TOL[odt] if name == "out" else (TOL[xdt] if name in ("dx", "dy") else GRAD_TOL)
+        assert rel_err(np_of(a), r, floor=1e-3) < tol, (name, rel_err(np_of(a), r))
+
+
+@pytest.mark.parametrize("T,n,C", [(900, 24, 20), (4000, 12, 7), (700, 40, 12)])
+def test_mxf32_many_slabs_per_wave(T, n, C, knobs):
+    """Two workgroups' worth of rows: every wave walks many slabs and the sums match the VALU kernels' (MHC_MIX32=0)."""
+    g = rng(9400 + T)
+    x, y, dout = (dev_tensor(g.standard_normal((T, n, C))) for _ in range(3))
+    M = dev_tensor(g.uniform(size=(n, n)))
+    res = []
+    for on in (1, 0):
+        knobs("MHC_MIX32", on)
+        knobs("MHC_MIX_FWD_GRID", 1)
+        knobs("MHC_MIX_BWD_GRID", 1)
+        ts = [t.clone().requires_grad_(True) for t in (x, M, y)]
+        out = ops.stream_mix_add_hip_autograd(*ts)
+        res.append([out.detach(), *torch.autograd.grad(out, ts, dout)])
+    for a, b in zip(*res):
+        assert rel_err(np_of(a), np_of(b)) < 1e-5
+    assert not torch.equal(res[0][2], res[1][2])
+
+
+def test_mxf32_unaligned_rows():
+    """Operands at addresses that are no multiple of four elements give the same values."""
+    T, n, C = 30, 12, 24
+    g = rng(9500)
+    vals = [dev_tensor(g.standard_normal((T, n, C))) for _ in range(3)]
+    hp, hq, hr, _ = (dev_tensor(v) for v in params(g, n, C))
+    res = []
+    for shift in (0, 1):
+        ts = []
+        for v in vals:
+            buf = torch.empty(v.numel() + 1, device="cuda")
+            t = buf[shift:shift + v.numel()].view(T, n, C)
+            ts.append(t.copy_(v))
+        xs, ys = (t.detach().requires_grad_(True) for t in ts[:2])
+        ps = [p.clone().requires_grad_(True) for p in (hp, hq, hr)]
+        out = ops.post_combine(xs, ys, *ps)
+        res.append([out.detach(), *torch.autograd.grad(out, [xs, ys, *ps], ts[2])])
+    for a, b in zip(*res):
+        assert rel_err(np_of(a), np_of(b)) < 1e-6
