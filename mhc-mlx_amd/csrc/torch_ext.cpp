@@ -1,4 +1,5 @@
-// Torch binding of libmhc_hip for MHCLayer's hot calls (mhc_mlx/layer.py:339-435).
+// Torch binding of libmhc_hip for MHCLayer's hot calls (mhc_mlx/layer.py:339-435), MHCRewire's pre-scale and
+// post-combine (layer.py:302-337, 469-492) and residual_add_agg (utils.py:4-24).
 //
 // The module's work per call is one or two library launches; at small batch
 // its latency is the host code around them.  This binding does that host code
@@ -221,6 +222,170 @@ at::Tensor layer_forward_nograd(const at::Tensor& x, const at::Tensor& hpre, con
                    at::Tensor()).first;
 }
 
+// ---------------------------------------------------------------------------
+// MHCRewire and residual_add_agg: the Python Functions of ops.py (which run
+// under a kernel timer) with their host steps in C++.  A training step of
+// MHCRewire around a Linear of 128 tokens is host-bound: 346 us through the
+// Python Functions and their ctypes calls, 240 us here (of which the Linear's
+// own forward and backward take 106 us); residual_add_agg of 16 tokens
+// without a gradient 13.9 against 7.3 us.
+// ---------------------------------------------------------------------------
+
+// t in the kernels' dtypes for a second operand of x's: x's dtype or fp32.
+at::Tensor like_x(const at::Tensor& t, at::ScalarType xt) {
+  const at::ScalarType st = t.scalar_type();
+  return (st == xt || st == at::kFloat ? t : t.to(at::kFloat)).contiguous();
+}
+
+void check_on(const at::Tensor& x, std::initializer_list<const at::Tensor*> ts) {
+  TORCH_CHECK_VALUE(x.is_cuda(), "the HIP path needs GPU tensors (got x on ", x.device(), ")");
+  for (const at::Tensor* t : ts)
+    TORCH_CHECK_VALUE(t->device() == x.device(), "every tensor must be on x's device ", x.device(), " (got ",
+                      t->device(), ")");
+}
+
+// x_pre = sigmoid(H_pre_raw)_i x_i; with `pass` x itself is returned too, for the post-combine, whose x gradient the VJP
+// adds into its own dx pass.
+struct StreamScaleFn : public torch::autograd::Function<StreamScaleFn> {
+  static variable_list forward(AutogradContext* ctx, const at::Tensor& x, const at::Tensor& hpre, bool pass) {
+    const at::Tensor xc = x.contiguous();
+    at::Tensor out = at::empty_like(xc);
+    const int xt = dtype_code(xc.scalar_type());
+    check(mhc_stream_scale_fwd(xc.data_ptr(), xt, fp(hpre), MHC_H_RAW, out.data_ptr(), xt, x.size(0), (int)x.size(1),
+                               (int)x.size(2), stream_of(xc)),
+          "mhc_stream_scale_fwd");
+    ctx->save_for_backward({x, hpre});
+    ctx->set_materialize_grads(false);
+    if (pass) return {out, x};
+    return {out};
+  }
+
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const auto sv = ctx->get_saved_variables();
+    const at::Tensor pass = grads.size() > 1 ? grads[1] : at::Tensor();
+    if (!grads[0].defined()) return {pass, at::Tensor(), at::Tensor()};
+    const at::Tensor x = sv[0].contiguous(), &hpre = sv[1];
+    const int64_t T = x.size(0);
+    const int n = (int)x.size(1), C = (int)x.size(2), xt = dtype_code(x.scalar_type());
+    const at::Tensor g = like_x(grads[0], x.scalar_type());
+    const at::Tensor acc = pass.defined() ? pass.to(x.scalar_type()).contiguous() : at::Tensor();
+    at::Tensor dx = at::empty_like(x), dpre = at::empty(hpre.sizes(), hpre.options());
+    const size_t nb = mhc_stream_scale_bwd_workspace_bytes(T, n, C);
+    at::Tensor ws = at::empty({(int64_t)std::max<size_t>(nb, 1)}, x.options().dtype(at::kByte));
+    check(mhc_stream_scale_bwd(x.data_ptr(), xt, g.data_ptr(), dtype_code(g.scalar_type()), fp(hpre), MHC_H_RAW,
+                               acc.defined() ? acc.data_ptr() : nullptr, dx.data_ptr(), xt, fp(dpre), ws.data_ptr(), nb,
+                               T, n, C, stream_of(x)),
+          "mhc_stream_scale_bwd");
+    return {dx, dpre, at::Tensor()};
+  }
+};
+
+variable_list stream_scale(const at::Tensor& x, const at::Tensor& hpre, bool pass) {
+  check_on(x, {&hpre});
+  TORCH_CHECK_VALUE(x.dim() == 3 && hpre.numel() == x.size(1), "x must be [B, n, C] and H_pre_raw [n]");
+  return StreamScaleFn::apply(x, f32(hpre), pass);
+}
+
+// out = H_post (y_inner + (M diag(H_pre)) x) from raw logits, M projected here; with `record` the projection records its
+// VJP state (n >= 16).
+struct PostCombineFn : public torch::autograd::Function<PostCombineFn> {
+  static at::Tensor forward(AutogradContext* ctx, const at::Tensor& x, const at::Tensor& y, const at::Tensor& hpre,
+                            const at::Tensor& hpost, const at::Tensor& hres, int64_t iters, double eps,
+                            int64_t out_code, bool record) {
+    const int64_t T = x.size(0);
+    const int n = (int)x.size(1), C = (int)x.size(2);
+    const at::Tensor xc = x.contiguous(), yc = like_x(y, x.scalar_type());
+    void* s = stream_of(xc);
+    at::Tensor state, M = at::empty_like(hres);
+    if (record && (n != 16 || reinterpret_cast<uintptr_t>(hres.data_ptr()) % 16 == 0)) {
+      const size_t nst = mhc_sinkhorn_state_bytes(1, n, (int)iters);
+      if (nst > 0) state = at::empty({(int64_t)nst}, x.options().dtype(at::kByte));
+    }
+    if (state.defined())
+      check(mhc_sinkhorn_fwd_record(fp(hres), fp(M), state.data_ptr(), (size_t)state.numel(), 1, n, (int)iters,
+                                    (float)eps, s),
+            "mhc_sinkhorn_fwd_record");
+    else
+      check(mhc_sinkhorn_fwd(fp(hres), fp(M), 1, n, (int)iters, (float)eps, s), "mhc_sinkhorn_fwd");
+    const at::ScalarType ot = out_code == MHC_DTYPE_F32 ? at::kFloat : x.scalar_type();
+    at::Tensor out = at::empty({T, n, C}, x.options().dtype(ot));
+    check(mhc_stream_mix_add_fwd(xc.data_ptr(), dtype_code(xc.scalar_type()), yc.data_ptr(),
+                                 dtype_code(yc.scalar_type()), fp(M), fp(hpre), fp(hpost), MHC_H_RAW, out.data_ptr(),
+                                 dtype_code(ot), T, n, C, s),
+          "mhc_stream_mix_add_fwd");
+    ctx->save_for_backward({x, y, hpre, hpost, hres, M, state});
+    ctx->saved_data["iters"] = iters;
+    ctx->saved_data["eps"] = eps;
+    return out;
+  }
+
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const auto sv = ctx->get_saved_variables();
+    const at::Tensor x = sv[0].contiguous(), y = like_x(sv[1], x.scalar_type());
+    const at::Tensor &hpre = sv[2], &hpost = sv[3], &hres = sv[4], &M = sv[5], &state = sv[6];
+    const int64_t T = x.size(0);
+    const int n = (int)x.size(1), C = (int)x.size(2), iters = (int)ctx->saved_data["iters"].toInt();
+    const float eps = (float)ctx->saved_data["eps"].toDouble();
+    const at::Tensor g = like_x(grads[0], x.scalar_type());
+    at::Tensor dx = at::empty_like(x), dy = at::empty_like(y);
+    // the three parameter gradients and dM in one allocation, each starting on a 256-byte boundary
+    auto up = [](int64_t v) { return (v + 63) / 64 * 64; };
+    const int64_t o1 = up(n), o2 = o1 + up(n), o3 = o2 + up((int64_t)n * n);
+    at::Tensor pg = at::empty({o3 + (int64_t)n * n}, hres.options());
+    at::Tensor dpre = pg.narrow(0, 0, n).view(hpre.sizes()), dpost = pg.narrow(0, o1, n).view(hpost.sizes());
+    at::Tensor dres = pg.narrow(0, o2, (int64_t)n * n).view(hres.sizes());
+    float* dM = fp(pg) + o3;
+    const int xt = dtype_code(x.scalar_type()), yt = dtype_code(y.scalar_type());
+    void* s = stream_of(x);
+    // one workspace: the post-combine's VJP, then the projection's
+    const size_t nmix = mhc_stream_mix_add_bwd_workspace_bytes(T, n, C);
+    const size_t nsk = state.defined() ? 0 : mhc_sinkhorn_bwd_workspace_bytes(1, n, iters);
+    at::Tensor ws = at::empty({(int64_t)std::max<size_t>(std::max(nmix, nsk), 1)}, x.options().dtype(at::kByte));
+    check(mhc_stream_mix_add_bwd(x.data_ptr(), xt, y.data_ptr(), yt, g.data_ptr(), dtype_code(g.scalar_type()), fp(M),
+                                 fp(hpre), fp(hpost), MHC_H_RAW, dx.data_ptr(), xt, dy.data_ptr(), yt, dM, fp(dpre),
+                                 fp(dpost), ws.data_ptr(), nmix, T, n, C, s),
+          "mhc_stream_mix_add_bwd");
+    if (state.defined())
+      check(mhc_sinkhorn_bwd_recorded(fp(hres), dM, fp(dres), state.data_ptr(), (size_t)state.numel(), 1, n, iters, eps,
+                                      s),
+            "mhc_sinkhorn_bwd_recorded");
+    else
+      check(mhc_sinkhorn_bwd(fp(hres), dM, fp(dres), 1, n, iters, eps, nsk ? ws.data_ptr() : nullptr, nsk, s),
+            "mhc_sinkhorn_bwd");
+    return {dx, dy.scalar_type() == sv[1].scalar_type() ? dy : dy.to(sv[1].scalar_type()), dpre, dpost, dres,
+            at::Tensor(), at::Tensor(), at::Tensor(), at::Tensor()};
+  }
+};
+
+at::Tensor post_combine(const at::Tensor& x, const at::Tensor& y, const at::Tensor& hpre, const at::Tensor& hpost,
+                        const at::Tensor& hres, int64_t iters, double eps, int64_t out_code) {
+  check_on(x, {&y, &hpre, &hpost, &hres});
+  TORCH_CHECK_VALUE(x.dim() == 3 && y.sizes() == x.sizes(), "x and y_inner must be [B, n, C]");
+  const int64_t n = x.size(1);
+  TORCH_CHECK_VALUE(hpre.numel() == n && hpost.numel() == n && hres.numel() == n * n,
+                    "parameter sizes do not match x ", x.sizes());
+  const bool record = at::GradMode::is_enabled() && hres.requires_grad();
+  return PostCombineFn::apply(x, y, f32(hpre), f32(hpost), f32(hres), iters, eps, out_code, record);
+}
+
+// (x + res, sum_i H_pre[i] (x + res)[:, i]) for a call that needs no gradient; x and res of one dtype, out of
+// `out_code`'s.
+std::tuple<at::Tensor, at::Tensor> residual_add_agg_nograd(const at::Tensor& x, const at::Tensor& res,
+                                                           const at::Tensor& hpre, int64_t out_code) {
+  check_on(x, {&res, &hpre});
+  TORCH_CHECK_VALUE(x.dim() == 3 && res.sizes() == x.sizes() && x.scalar_type() == res.scalar_type() &&
+                        hpre.numel() == x.size(1),
+                    "x and res must be [B, n, C] of one dtype and H_pre [n]");
+  const int64_t T = x.size(0), C = x.size(2);
+  const at::Tensor xc = x.contiguous(), rc = res.contiguous(), hp = f32(hpre);
+  const at::ScalarType ot = out_code == MHC_DTYPE_BF16 ? at::kBFloat16 : out_code == MHC_DTYPE_F16 ? at::kHalf : at::kFloat;
+  at::Tensor out = at::empty({T, x.size(1), C}, x.options().dtype(ot)), y = at::empty({T, C}, x.options().dtype(at::kFloat));
+  check(mhc_residual_add_agg_fwd(xc.data_ptr(), rc.data_ptr(), dtype_code(xc.scalar_type()), fp(hp), MHC_H_ACTIVATED,
+                                 out.data_ptr(), dtype_code(ot), fp(y), T, (int)x.size(1), (int)C, stream_of(xc)),
+        "mhc_residual_add_agg_fwd");
+  return {out, y};
+}
+
 bool env_is_one(const char* name) {
   const char* v = std::getenv(name);
   return v != nullptr && v[0] == '1' && v[1] == '\0';
@@ -309,6 +474,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.doc() = "torch binding of libmhc_hip for MHCLayer's forward and backward";
   m.def("layer_apply", &layer_apply, "MHCLayer forward with its backward as a C++ autograd Function");
   m.def("layer_forward_nograd", &layer_forward_nograd, "MHCLayer forward without autograd");
+  m.def("stream_scale", &stream_scale, "MHCRewire's pre-scale (and x itself) with its backward in C++");
+  m.def("post_combine", &post_combine, "MHCRewire's post-combine from raw logits with its backward in C++");
+  m.def("residual_add_agg_nograd", &residual_add_agg_nograd, "residual_add_agg without autograd");
   m.def("module_forward", &module_forward, "MHCLayer.forward's accelerated path (None: take the general path)");
   m.def("module_call", &module_call, "module_forward with the arguments read from the MHCLayer instance");
 }

@@ -764,6 +764,9 @@ def post_combine(x, y_inner, H_pre_raw, H_post_raw, H_res_raw, sinkhorn_iters: i
     if out_dtype not in (torch.float32, x.dtype):
         raise ValueError(f"unsupported output_dtype: {output_dtype}")
     _require_gpu(x, y_inner, H_pre_raw, H_post_raw, H_res_raw)
+    if profiling._active is None and int(H_pre_raw.numel()) == n and int(H_post_raw.numel()) == n:
+        return _binding().post_combine(x, y_inner, H_pre_raw, H_post_raw, H_res_raw, int(sinkhorn_iters), float(eps),
+                                       _DTYPE_CODE[out_dtype])
     return PostCombineFn.apply(x, y_inner, H_pre_raw, H_post_raw, H_res_raw, int(sinkhorn_iters),
                                float(eps), out_dtype)
 
@@ -821,6 +824,8 @@ def _stream_scale_check(x, H_pre_raw):
 def stream_scale(x, H_pre_raw):
     """Pre-scale of MHCRewire: [B, n, C] * sigmoid(H_pre_raw)[n]."""
     _stream_scale_check(x, H_pre_raw)
+    if profiling._active is None:
+        return _binding().stream_scale(x, H_pre_raw, False)[0]
     return StreamScaleFn.apply(x, H_pre_raw, False)
 
 
@@ -828,6 +833,8 @@ def stream_scale_and_pass(x, H_pre_raw):
     """(stream_scale(x, H_pre_raw), x): the second output is x for a second use (MHCRewire's
     post-combine) whose gradient the pre-scale's VJP adds into dx in its own pass."""
     _stream_scale_check(x, H_pre_raw)
+    if profiling._active is None:
+        return tuple(_binding().stream_scale(x, H_pre_raw, True))
     return StreamScaleFn.apply(x, H_pre_raw, True)
 
 
@@ -920,4 +927,7 @@ def residual_add_agg_hip(x, res, H_pre, threads_per_group=None, output_dtype=Non
     else:
         raise ValueError(f"unsupported output_dtype: {output_dtype}")
     _require_gpu(x, res, H_pre)
+    if (profiling._active is None and x.dtype == res.dtype and not _needs_grad(x, res, H_pre)
+            and torch.autograd.forward_ad._current_level < 0):  # (forward mode is refused by the Function)
+        return _binding().residual_add_agg_nograd(x, res, H_pre, _DTYPE_CODE[out_dtype])
     return ResidualAddAggFn.apply(x, res, H_pre, out_dtype)

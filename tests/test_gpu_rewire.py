@@ -433,3 +433,36 @@ def test_post_combine_generic_mfma_sums(B, n, C, xdt, gdt, odt, knobs):
     assert torch.equal(got[1], valu[1]) and torch.equal(got[2], valu[2])
     for name, a, b in zip(names[2:], got[3:], valu[3:]):
         assert rel_err(np_of(a), np_of(b)) < 1e-5, name
+
+
+@pytest.mark.parametrize("n,xdt,ydt,pdt", [(4, "bf16", "bf16", "f32"), (16, "f16", "f32", "f32"), (20, "bf16", "f16", "f32"),
+                                           (33, "f32", "f32", "bf16")])
+def test_rewire_binding_matches_the_python_functions(n, xdt, ydt, pdt):
+    """The pre-scale, the post-combine and residual_add_agg through the C++ binding are bitwise the Python Functions
+    (which run under a kernel timer): y of x's dtype, fp32 or the other half type, parameters in fp32 or bf16, a
+    non-contiguous x, and one of the pre-scale's two outputs unused."""
+    from mhc_mlx_amd import profiling, residual_add_agg
+
+    T, C = 37, 24
+    g = rng(880 + n)
+    x = dev_tensor(g.standard_normal((n, T, C)), xdt).transpose(0, 1)
+    y = dev_tensor(g.standard_normal((T, n, C)), ydt)
+    dout = dev_tensor(g.standard_normal((T, n, C)))
+    hpre, hpost, hres, _ = (dev_tensor(v, pdt) for v in params(g, n, C))
+
+    def run():
+        xs, ys = (t.detach().requires_grad_(True) for t in (x, y))
+        ps = [t.detach().requires_grad_(True) for t in (hpre, hpost, hres)]
+        pre, xp = ops.stream_scale_and_pass(xs, ps[0])
+        out = ops.post_combine(xp, ys, *ps)
+        both = torch.autograd.grad([pre, out], [xs, ys, *ps], [dout.to(pre.dtype), dout], retain_graph=True)
+        only = torch.autograd.grad(out, [xs, ps[2]], dout)
+        with torch.no_grad():
+            res = residual_add_agg(x, y.to(x.dtype), hpre.float())
+        return [pre.detach(), out.detach(), *both, *only, ops.stream_scale(x, hpre).detach(), *res]
+
+    a = run()
+    with profiling.kernel_timer():
+        b = run()
+    for u, v in zip(a, b):
+        assert u.dtype == v.dtype and u.shape == v.shape and torch.equal(u, v)
