@@ -22,6 +22,7 @@
 #include "mhc_device.hpp"
 #include "mhc_generic.hpp"
 #include "mhc_lf32.hpp"
+#include "mhc_lv.hpp"
 #include "mhc_mfma32.hpp"
 #include "mhc_host.hpp"
 #include "mhc_plan.hpp"
@@ -1646,6 +1647,23 @@ int launch_bwd_tile(BwdArgs A, const BwdLayout& L, int64_t* num_partials, hipStr
   return MHC_OK;
 }
 
+// Whether fused_bwd_lw_kernel is asked before the narrow-token kernel of lv.hpp (each takes what the other declines).
+// Measured, backward kernel, lw against lv: layer-wide 16-bit rows of 2048 channels and more stream better on one
+// workgroup per token with its sums in registers (32768 x 4 x 4096 bf16 567 against 660 us, 8192 x 8 x 4096 365 against
+// 431 us; at C = 1024 163 against 147 us and 165 against 154 us, at C = 512 101 against 72 us); so do fp32 rows of 513 to
+// 1024 channels at n <= 4 (10000 x 4 x 1000 90 against 96 us; 8192 x 4 x 4096 280 against 276 us) and per-token 16-bit
+// rows of 1025 to 2048 channels at n = 8 (281 against 316 us).  Partial chunks per token, which lw would walk on the tile
+// kernel, all go to lv (4882 x 2 x 4096 fp32 210 against 89 us).
+template <int NMAX, typename XT, typename GT, bool PT>
+bool lw_first(const BwdArgs& A) {
+  const bool pair16 = std::is_same<XT, GT>::value && sizeof(XT) == 2;
+  if (pair16) {
+    if (PT) return NMAX == 8 && A.n == NMAX && A.C > 1024 && A.C <= 2048;
+    return A.n == NMAX && A.C >= 2048;
+  }
+  return NMAX <= 4 && sizeof(XT) == 4 && A.C > 512 && A.C <= 1024 && (!PT || A.n == NMAX);
+}
+
 template <int NMAX, typename XT, typename GT, bool PT>
 int launch_bwd(BwdArgs A, const BwdLayout& L, int64_t* num_partials, hipStream_t stream) {
   if constexpr (!PT && NMAX == 16 && std::is_same<XT, GT>::value && ElemTraits<XT>::kBytes == 2) {
@@ -1659,9 +1677,13 @@ int launch_bwd(BwdArgs A, const BwdLayout& L, int64_t* num_partials, hipStream_t
     if (rc != 1) return rc;
   }
   if constexpr (NMAX <= 8) {
-    const int legacy = knob(kKnobBwdLegacy, 0);
-    if (!legacy) {
-      const int rc = launch_bwd_lw<NMAX, XT, GT, PT>(A, L, num_partials, stream);
+    if (!knob(kKnobBwdLegacy, 0)) {
+      const bool lw = lw_first<NMAX, XT, GT, PT>(A);
+      int rc = lw ? launch_bwd_lw<NMAX, XT, GT, PT>(A, L, num_partials, stream) : 1;
+      if (rc != 1) return rc;
+      rc = lv_fused_bwd(gen_args(A, L), dtype_code<XT>(), dtype_code<GT>(), L.gmax, stream, num_partials);
+      if (rc != 1) return rc;
+      rc = lw ? 1 : launch_bwd_lw<NMAX, XT, GT, PT>(A, L, num_partials, stream);
       if (rc != 1) return rc;
     }
   }

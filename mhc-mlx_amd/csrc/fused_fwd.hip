@@ -17,6 +17,7 @@
 #include "mhc_device.hpp"
 #include "mhc_generic.hpp"
 #include "mhc_lf32.hpp"
+#include "mhc_lv.hpp"
 #include "mhc_mfma32.hpp"
 #include "mhc_host.hpp"
 #include "mhc_plan.hpp"
@@ -677,6 +678,17 @@ int launch_fwd(FwdArgs A, hipStream_t stream) {
   if constexpr (!PT && NMAX <= 8) {
     const int rc = launch_fwd_full<NMAX, XT, OT>(A, stream);
     if (rc != 1) return rc;
+  }
+  // What whole workgroups of whole chunks do not cover goes to the narrow-token kernel (forward, this kernel against
+  // it: 9990 x 4 x 1001 bf16 103 against 36 us, 32768 x 4 x 96 bf16 37 against 14 us, per token 8192 x 4 x 4096 fp32 216
+  // against 186 us), except at n > 4 with whole vectors where that one would read x twice (625 x 8 x 8000 bf16 44
+  // against 52 us) or its lanes run out of work against a token's 80 parameters (per token, 16-bit output: 5000 x 8 x
+  // 1000 37 against 41 us).
+  if constexpr (NMAX <= 8) {
+    if (!(A.vec && A.n > 4 && (A.C > 4096 || (PT && ElemTraits<OT>::kBytes == 2)))) {
+      const int rc = lv_fused_fwd(gen_args(A), dtype_code<XT>(), dtype_code<OT>(), stream);
+      if (rc != 1) return rc;
+    }
   }
   if constexpr (NMAX == 16) {
     int rc = launch_fwd_mfma16<XT, OT, PT>(A, stream);

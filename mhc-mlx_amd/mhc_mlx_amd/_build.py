@@ -25,6 +25,7 @@ OFFLOAD_ARCH = os.environ.get("MHC_OFFLOAD_ARCH", "gfx950")
 SOURCES = ["capi.hip", "sinkhorn.hip", "fused_fwd.hip", "fused_bwd.hip", "stream_mix.hip", "generic.hip", "residual.hip",
            "mfma32.hip", "mix32.hip", "lf32_fwd.hip",
            "lf32_bwd_f32.hip", "lf32_bwd_bf16.hip", "lf32_bwd_f16.hip", "mxf32_f32.hip", "mxf32_bf16.hip", "mxf32_f16.hip",
+           "lv_fwd_f32.hip", "lv_fwd_bf16.hip", "lv_fwd_f16.hip", "lv_bwd_f32.hip", "lv_bwd_bf16.hip", "lv_bwd_f16.hip",
            "noalloc.hip"]
 
 # Packed-FP32 VALU forms are disabled for every device pass (hipcc only; the

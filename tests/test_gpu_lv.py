@@ -1,0 +1,78 @@
+"""GPU parity of the narrow-token layer kernels (csrc/lv.hpp, n <= 8) against the float64 oracle.
+
+They take tokens that are no whole workgroup of whole aligned chunks.  The sizes sit at the edges of their splits: 16, 32
+and 64 lanes per token, one wave and several, one to four chunks per wave, the two-pass form, rows taken one, four and
+eight elements at a time, n below its 2, 4 or 8 slots, and a last workgroup that is not full.
+"""
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import mhc_oracle as O
+from tests._helpers import GRAD_TOL, TOL, dev_tensor, np_of, params, rel_err, rng, to_dtype_np
+
+from mhc_mlx_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+EPS = 1e-5
+SHAPES = [(37, 2, 1), (19, 3, 16), (70, 4, 64), (33, 4, 65), (18, 8, 100), (9, 5, 128), (21, 1, 132), (5, 2, 300),
+          (7, 4, 777), (3, 6, 1000), (6, 4, 1040), (4, 8, 1030), (3, 2, 2056), (2, 3, 4100), (2, 8, 2500), (3, 4, 8008),
+          (2, 4, 9001), (2, 7, 4200)]
+
+
+@pytest.mark.parametrize("T,n,C", SHAPES)
+@pytest.mark.parametrize("xdt,odt", [("f32", "f32"), ("bf16", "f32"), ("f16", "f16"), ("bf16", "bf16")])
+@pytest.mark.parametrize("per_token", [False, True])
+@pytest.mark.parametrize("grid", [None, 1])
+def test_lv_forward_and_backward(T, n, C, xdt, odt, per_token, grid, knobs):
+    """Output and every gradient, on the whole chip and on one workgroup (per CU) that walks every token; reruns are
+    bitwise equal."""
+    if grid is not None:
+        knobs("MHC_FWD_GRID", grid)
+        knobs("MHC_BWD_GRID", grid)
+    g = rng(9700 + T + n + C)
+    x, dout = to_dtype_np(g.standard_normal((T, n, C)), xdt), to_dtype_np(g.standard_normal((T, n, C)), odt)
+    ps = params(g, n, C, per_token_B=T if per_token else None)
+    fn = ops.mhc_layer_forward_dynamic if per_token else ops.mhc_layer_forward
+
+    def run():
+        xt = dev_tensor(x, xdt).requires_grad_(True)
+        pt = [dev_tensor(v).requires_grad_(True) for v in ps]
+        out = fn(xt, *pt, sinkhorn_iters=20, eps=EPS, output_dtype=None if odt == "f32" else xt.dtype)
+        return [out.detach(), *torch.autograd.grad(out, [xt, *pt], dev_tensor(dout, odt))]
+
+    got, again = run(), run()
+    for a, b in zip(got, again):
+        assert torch.equal(a, b)
+    refs = [O.mhc_forward_reference(x, *ps, sinkhorn_iters=20, eps=EPS),
+            *O.mhc_backward_reference(x, *ps, dout, sinkhorn_iters=20, eps=EPS)]
+    for name, a, r in zip(("out", "dx", "dH_pre", "dH_post", "dH_res", "d_w"), got, refs):
+        tol = TOL[odt] if name == "out" else (TOL[xdt] if name == "dx" else GRAD_TOL)
+        # dH_pre: at n = 1, and with one channel, the output does not depend on H_pre (the RMS norm undoes its scale) and
+        # dH_pre is a difference of terms of the size of the sums behind it, about sqrt(T n C)
+        floor = np.sqrt(T * n * C) if name == "dH_pre" and (n == 1 or C == 1) else 1e-3
+        assert rel_err(np_of(a), r, floor=floor) < tol, (name, rel_err(np_of(a), r, floor=floor))
+
+
+@pytest.mark.parametrize("n,C", [(4, 100), (8, 516), (3, 2000)])
+def test_lv_matches_the_tile_kernel(n, C, knobs):
+    """The same gradients as the tile kernel (MHC_BWD_LEGACY=1) to fp32 summation order, from operands whose addresses are
+    no multiple of four elements too."""
+    T = 50
+    g = rng(9800 + n)
+    x, dout = (dev_tensor(g.standard_normal((T, n, C))) for _ in range(2))
+    ps = [dev_tensor(v) for v in params(g, n, C)]
+    res = []
+    for legacy, shift in ((0, 0), (0, 1), (1, 0)):
+        knobs("MHC_BWD_LEGACY", legacy)
+        buf = torch.empty(x.numel() + 1, device="cuda")
+        xs = buf[shift:shift + x.numel()].view(T, n, C).copy_(x).detach().requires_grad_(True)
+        pt = [p.clone().requires_grad_(True) for p in ps]
+        out = ops.mhc_layer_forward(xs, *pt, eps=EPS)
+        res.append([out.detach(), *torch.autograd.grad(out, [xs, *pt], dout)])
+    for other in res[1:]:
+        for a, b in zip(res[0], other):
+            assert rel_err(np_of(a), np_of(b)) < 1e-5
+    assert not all(torch.equal(a, b) for a, b in zip(res[0][1:], res[2][1:]))
