@@ -26,15 +26,16 @@
 // SPW > 0 (layer-wide, n <= 32): M^T g of the wave's SPW slabs is held across
 // the barrier and the next token's x and g are loaded meanwhile.  SPW = 0: the
 // wave walks any number of slabs, y and d in LDS, and reads g again after the
-// barrier (from the caches).  Per-token parameters take SPW = 0 with one wave
-// per workgroup, so the token's dM, dA and dP are the wave's own.  Above
+// barrier (from the caches).  Per-token parameters take SPW = 0, with one wave
+// per workgroup where there are tokens enough to fill the chip (the token's
+// dM, dA and dP are then the wave's own), else up to four.  Above
 // n = 32 (BIG) M^T's operands come from LDS, one 16-row block at a time.
 //
 // Backward kernel, against the VALU kernels before it: 4096 x 32 x 512 fp32
 // 1355 -> 161 us (5.0 TB/s), 4096 x 16 x 1024 fp32 393 -> 140 us (5.8 TB/s),
 // 2048 x 64 x 512 fp32 4145 -> 298 us (one wave per SIMD: dM alone is 64
 // registers), 1024 x 32 x 4096 fp32 3214 -> 400 us, per token 4096 x 32 x 512
-// fp32 1371 -> 180 us, 3001 x 16 x 1100 fp16 371 -> 101 us and 20000 x 24 x 100
+// fp32 1371 -> 190 us and 2500 x 10 x 4000 fp32 479 us (758 us on one wave a token), 3001 x 16 x 1100 fp16 371 -> 101 us and 20000 x 24 x 100
 // bf16 1989 -> 133 us (16-bit rows: bound by the VALU's conversions and LDS).
 #pragma once
 
@@ -51,13 +52,14 @@ namespace mhc {
 namespace {
 
 constexpr int kLfPitch = kLfSlab + 4;
+constexpr int kLfPtWaves = 4;  // waves per token at most with per-token parameters
 // floats of one wave's LDS: x rows, g rows, and y, d w, y w of a slab
 constexpr int lf_wave_floats(int nb) { return 2 * 16 * nb * kLfPitch + 3 * kLfSlab; }
 // floats of M^T's operands (BIG)
 constexpr int lf_mat_floats(int nb) { return nb > 2 ? nb * nb * 256 + 16 * nb : 0; }
 
 template <typename XT, typename GT, int NB, int SPW, int MODE, bool PT>
-__global__ __launch_bounds__(PT ? 64 : (NB > 2 ? 256 : 64 * kLfMaxWaves)) void lf32_bwd_kernel(GenArgs A) {
+__global__ __launch_bounds__(PT ? 64 * kLfPtWaves : (NB > 2 ? 256 : 64 * kLfMaxWaves)) void lf32_bwd_kernel(GenArgs A) {
   constexpr bool VEC = MODE != kLfElem;
   constexpr int NK = 4 * NB;
   constexpr int NJ = SPW > 0 ? SPW : 1;
@@ -304,6 +306,30 @@ __global__ __launch_bounds__(PT ? 64 : (NB > 2 ? 256 : 64 * kLfMaxWaves)) void l
     }
   };
 
+  // the wave's dM, dA and dP into its LDS, and their sum over the waves (entry k of [dM n*n | dA n | dP n])
+  constexpr int NM = 256 * NB * NB;
+  auto spill_sums = [&] {
+    issue_fence();  // the wave's rows in LDS are done with
+#pragma unroll
+    for (int I = 0; I < NB; ++I) {
+#pragma unroll
+      for (int J = 0; J < NB; ++J)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) sx[(16 * I + 4 * q + k) * (16 * NB) + 16 * J + r] = dm[I][J][k];
+      const float va = lf_sum_q(da[I]), vp = lf_sum_q(dp[I]);
+      if (q == 0) {
+        sx[NM + 16 * I + r] = va;
+        sx[NM + 16 * NB + 16 * I + r] = vp;
+      }
+    }
+  };
+  auto wave_total = [&](int k) {
+    const int at = k < nn ? (k / n) * (16 * NB) + k % n : (k < nn + n ? NM + k - nn : NM + 16 * NB + k - nn - n);
+    float v = 0.0f;
+    for (int wv = 0; wv < nw; ++wv) v += lf_smem[wv * lf_wave_floats(NB) + at];
+    return v;
+  };
+
   int it = 0;
   float dwr[NJ][4];
   if constexpr (SPW > 0) {
@@ -408,30 +434,24 @@ __global__ __launch_bounds__(PT ? 64 : (NB > 2 ? 256 : 64 * kLfMaxWaves)) void l
       if constexpr (PT) load_mat(t);
       rms(ss, sr, it);
       if constexpr (PT) {
-        const auto rm = lf_rsrc(A.dM_tok + t * (int64_t)nn, (uint32_t)nn * 4u);
-#pragma unroll
-        for (int I = 0; I < NB; ++I) {
-#pragma unroll
-          for (int J = 0; J < NB; ++J)
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-              const int i = 16 * I + 4 * q + k, j = 16 * J + r;
-              const float v = dm[I][J][k];  // a scalar before the bit cast
-              __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), rm,
-                                                    i < n && j < n ? (uint32_t)(i * n + j) * 4u : kLfOut, 0, 0);
+        // the waves' parts through their slab rows (done with until the next token), added in wave order
+        spill_sums();
+        lds_barrier();
+        for (int k = threadIdx.x; k < nn + 2 * n; k += blockDim.x) {
+          float v = wave_total(k);
+          if (k < nn) {
+            A.dM_tok[t * nn + k] = v;
+          } else {
+            const bool post = k >= nn + n;
+            const int i = k - nn - (post ? n : 0);
+            if (raw) {
+              const float sg = sigmoidf_((post ? A.hpost : A.hpre)[t * A.h_ts + i]);
+              v *= (post ? 2.0f : 1.0f) * sg * (1.0f - sg);
             }
-          const int i = 16 * I + r;
-          float va = lf_sum_q(da[I]), vp = lf_sum_q(dp[I]);
-          const float ai = lf_lane(av, i), pi = lf_lane(pv, i);
-          if (raw) {
-            va *= ai * (1.0f - ai);
-            vp *= pi * (1.0f - 0.5f * pi);
-          }
-          if (q == 0 && i < n) {
-            A.dpre_tok[t * n + i] = va;
-            A.dpost_tok[t * n + i] = vp;
+            (post ? A.dpost_tok : A.dpre_tok)[t * n + i] = v;
           }
         }
+        lds_barrier();
       }
       for (int s = wave; s < S; s += nw) {
         float dy[4], w[4];
@@ -496,35 +516,21 @@ __global__ __launch_bounds__(PT ? 64 : (NB > 2 ? 256 : 64 * kLfMaxWaves)) void l
     for (int c = threadIdx.x; c < A.Cp; c += blockDim.x) prow[c] = c < C ? s_dw[c] : 0.0f;
   }
   if constexpr (!PT) {
-    issue_fence();  // the wave's rows in LDS are done with
-    constexpr int NM = 256 * NB * NB;
-#pragma unroll
-    for (int I = 0; I < NB; ++I) {
-#pragma unroll
-      for (int J = 0; J < NB; ++J)
-#pragma unroll
-        for (int k = 0; k < 4; ++k) sx[(16 * I + 4 * q + k) * (16 * NB) + 16 * J + r] = dm[I][J][k];
-      const float va = lf_sum_q(da[I]), vp = lf_sum_q(dp[I]);
-      if (q == 0) {
-        sx[NM + 16 * I + r] = va;
-        sx[NM + 16 * NB + 16 * I + r] = vp;
-      }
-    }
+    spill_sums();
     __syncthreads();
-    for (int k = threadIdx.x; k < nn + 2 * n; k += blockDim.x) {
-      const int at = k < nn ? (k / n) * (16 * NB) + k % n : (k < nn + n ? NM + k - nn : NM + 16 * NB + k - nn - n);
-      float v = 0.0f;
-      for (int wv = 0; wv < nw; ++wv) v += lf_smem[wv * lf_wave_floats(NB) + at];
-      prow[A.Cp + k] = v;
-    }
+    for (int k = threadIdx.x; k < nn + 2 * n; k += blockDim.x) prow[A.Cp + k] = wave_total(k);
   }
+}
+
+// bytes of a workgroup's LDS; `loop`: SPW = 0
+inline size_t lf_bwd_smem(int nb, int waves, int S, bool loop) {
+  return ((size_t)waves * lf_wave_floats(nb) + lf_mat_floats(nb) + (loop ? (size_t)3 * S * kLfSlab : 0)) * sizeof(float);
 }
 
 template <typename XT, typename GT, int NB, int SPW, int MODE, bool PT>
 int lf_bwd_launch(const GenArgs& A, int waves, int64_t gmax, hipStream_t s, int64_t* num_partials) {
   const int S = (int)ceil_div(A.C, kLfSlab);
-  const size_t smem =
-      ((size_t)waves * lf_wave_floats(NB) + lf_mat_floats(NB) + (SPW > 0 ? 0 : (size_t)3 * S * kLfSlab)) * sizeof(float);
+  const size_t smem = lf_bwd_smem(NB, waves, S, SPW == 0);
   const void* kfn = (const void*)lf32_bwd_kernel<XT, GT, NB, SPW, MODE, PT>;
   const int occ = occupancy_blocks(kfn, waves * 64, smem);
   if (occ <= 0) return 1;
@@ -553,8 +559,20 @@ template <typename XT, typename GT, int NB, int MODE>
 int lf_bwd_split(const GenArgs& A, int64_t gmax, hipStream_t s, int64_t* np) {
   const int S = (int)ceil_div(A.C, kLfSlab);
   if (A.M_ts != 0) {
-    if (lf_bwd_waves<NB>(A.C, 1) == 0) return 1;
-    return lf_bwd_launch<XT, GT, NB, 0, MODE, true>(A, 1, gmax, s, np);
+    // waves per token: the fewest with which eight waves can be resident on a CU (a workgroup's y, d and dw take 12 C
+    // bytes of LDS beside its waves' rows) and the tokens fill eight on every CU; else the most resident ones
+    int waves = 0;
+    int64_t best = 0;
+    for (int w = 1; w <= std::min(S, kLfPtWaves) && best < 8; ++w) {
+      const int64_t resident = w * (int64_t)(kLfLds / lf_bwd_smem(NB, w, S, true));
+      const int64_t filled = std::min(resident, ceil_div(A.T * w, (int64_t)device_cu_count()));
+      if (filled > best) {
+        best = filled;
+        waves = w;
+      }
+    }
+    if (waves == 0) return 1;
+    return lf_bwd_launch<XT, GT, NB, 0, MODE, true>(A, waves, gmax, s, np);
   }
   if constexpr (NB <= 2) {
     if (S <= kLfMaxWaves) return lf_bwd_launch<XT, GT, NB, 1, MODE, false>(A, S, gmax, s, np);
