@@ -450,6 +450,8 @@ __global__ __launch_bounds__(64 * kLvMaxWaves) void lv_bwd_kernel(GenArgs A, int
     float o[kRows ? 1 : NMAX][V], dy[V];
 #pragma unroll
     for (int v = 0; v < V; ++v) {
+      // 16-bit x with fp32 gradients at n = 8: one channel's products at a time, or the unpacked rows of all spill
+      if constexpr (NMAX > 4 && sizeof(XT) == 2 && sizeof(GT) == 4) __builtin_amdgcn_sched_barrier(0);
       float y, d;
       yd(j, v, y, d);
       const float yi = y * inv;
@@ -803,12 +805,17 @@ int lv_bwd_typed(const GenArgs& A, int64_t gmax, hipStream_t s, int64_t* np) {
       } else {
       const bool pt = A.M_ts != 0;
       return lv_by_split<MODE, lv_most(MODE, NM, true)>(A.C, pt, !pt, [&](auto sp, auto gr, int wpt) {
-        constexpr int SPW = decltype(sp)::value, G = decltype(gr)::value, V = lv_width(MODE);
-        if constexpr (NM > 4 && MODE == kLvElem && SPW == 0 && OCT) {
+        constexpr int G = decltype(gr)::value, V = lv_width(MODE);
+        if constexpr (NM > 4 && MODE == kLvElem && decltype(sp)::value == 0 && OCT) {
           return 1;  // (one offset per element of two 16-bit operands over eight streams: too many registers)
         } else {
           auto go = [&](auto ptc) {
             constexpr bool PT = decltype(ptc)::value;
+            // fp16 x, fp32 gradients, per-token parameters of n = 8: a lane's chunk does not stay in registers from the
+            // dot products to the gradients, so it is read again
+            constexpr bool kAgain = PT && NM > 4 && decltype(sp)::value == 1 && MODE != kLvElem && std::is_same<XT, _Float16>::value &&
+                                    sizeof(GT) == 4;
+            constexpr int SPW = kAgain ? 0 : decltype(sp)::value;
             const int tpb = lv_threads(wpt);
             const size_t chunk = (size_t)ceil_div(A.C, G * V) * G * V * sizeof(float);
             const size_t smem = SPW == 0 ? chunk * (wpt > 1 ? 1 : tpb / 64)

@@ -56,6 +56,13 @@ def test_lv_forward_and_backward(T, n, C, xdt, odt, per_token, grid, knobs):
         assert rel_err(np_of(a), r, floor=floor) < tol, (name, rel_err(np_of(a), r, floor=floor))
 
 
+@pytest.mark.parametrize("T,n,C", [(18, 8, 100), (9, 5, 128), (5, 8, 252), (4, 8, 1028), (3, 7, 1030), (2, 8, 2500)])
+@pytest.mark.parametrize("per_token", [False, True])
+def test_lv_f16_with_f32_output(T, n, C, per_token, knobs):
+    """fp16 streams with fp32 outputs at 4 < n <= 8, where the backward reads its rows a second time."""
+    test_lv_forward_and_backward(T, n, C, "f16", "f32", per_token, None, knobs)
+
+
 @pytest.mark.parametrize("n,C", [(4, 100), (8, 516), (3, 2000)])
 def test_lv_matches_the_tile_kernel(n, C, knobs):
     """The same gradients as the tile kernel (MHC_BWD_LEGACY=1) to fp32 summation order, from operands whose addresses are
