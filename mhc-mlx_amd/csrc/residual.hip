@@ -6,11 +6,11 @@
 //   d_val_i = dout_i + a_i dy                    dx = dres = d_val
 //   dh_pre_i = sum_{t,c} dy (x_i + res_i)
 //
-// HBM-bound streaming.  Work item = (token, chunk of V = 8 channels) over all
-// n streams, one item per thread (grid-stride beyond 2^24 blocks).  The streams are
-// visited in groups of G: the group's x and res chunks (2G 16-byte loads for
-// 16-bit types) are all issued before the first add, so every thread keeps
-// 2G loads in flight.  The backward splits the streams over grid.y (one
+// HBM-bound streaming.  Work item = (token, chunk of V channels) over all
+// n streams (grid-stride beyond 2^24 blocks).  The streams are
+// visited in groups of G: the group's x and res chunks are all issued before
+// the first add, so every thread keeps 2G loads in flight.  The backward takes
+// V = 8 channels per item and splits the streams over grid.y (one
 // group of 4 per block row) and writes one partial row of dh_pre per block,
 // finished by the fixed-order row reduction (deterministic, no atomics).
 #include "mhc_device.hpp"
@@ -62,9 +62,42 @@ MHC_DEV void store_c(T* p, const float (&v)[kResV], bool vec, int valid) {
   else store_partial<T, kResV>(p, v, valid);
 }
 
-template <int G, typename XT, typename OT>
+// V values to p (aligned to min(16, V elements)) as one store; NT: rows of whole 128-byte lines, past the caches.
+template <typename T, int V, bool NT>
+MHC_DEV void res_store(T* p, const float (&v)[V]) {
+  if constexpr (NT) {
+    store_vec<T, V, true>(p, v);
+  } else if constexpr (V == 1) {
+    store1<T>(p, v[0]);
+  } else {
+    constexpr int W = V * ElemTraits<T>::kBytes / 4;
+    uint32_t w[W];
+#pragma unroll
+    for (int k = 0; k < W; ++k) {
+      if constexpr (ElemTraits<T>::kBytes == 4) w[k] = __builtin_bit_cast(uint32_t, v[k]);
+      else w[k] = pack2<T>(v[2 * k], v[2 * k + 1]);
+    }
+    uint32_t* b = reinterpret_cast<uint32_t*>(p);
+    if constexpr (W == 2) {
+      const u32x2 u = {w[0], w[1]};
+      *reinterpret_cast<u32x2*>(b) = u;
+    } else {
+#pragma unroll
+      for (int k = 0; k < W; k += 4) st16<false>(b + k, w[k], w[k + 1], w[k + 2], w[k + 3]);
+    }
+  }
+}
+
+// Bound by HBM.  A lane takes V channels of every stream, so that one instruction of a wave reads or writes one
+// contiguous span: V = 8 when all rows are 16-bit, 4 when one is fp32 (eight channels of it are two 16-byte words,
+// and each instruction then covers every other 16 bytes), both for rows that keep the vectors aligned; V = 1, K
+// items a block apart, for the rest.  Against V = 8 for all, with ragged rows element by element: 8192 x 4 x 4096
+// bf16 to fp32 231 -> 192 us (6.3 TB/s), fp32 323 -> 285, bf16 to bf16 158 -> 152; 3000 x 16 x 1100 fp16 to fp32
+// 262 -> 92, 8000 x 4 x 1002 fp32 191 -> 79, 3001 x 7 x 1001 fp16 to fp32 111 -> 42.  K = 2 in groups of eight
+// streams, where K = 4 takes 256 registers: the last 42 us against 59.
+template <int G, typename XT, typename OT, int V, bool NT>
 __global__ __launch_bounds__(kResThreads) void residual_add_agg_kernel(ResArgs A) {
-  constexpr int V = kResV;
+  constexpr int K = V > 1 ? 1 : G > 4 ? 2 : 4;
   __shared__ float s_a[MHC_MAX_N];
   for (int i = threadIdx.x; i < A.n; i += blockDim.x) s_a[i] = act_pre(A, i);
   __syncthreads();
@@ -73,40 +106,50 @@ __global__ __launch_bounds__(kResThreads) void residual_add_agg_kernel(ResArgs A
   const XT* X = (const XT*)A.x;
   const XT* R = (const XT*)A.res;
   OT* O = (OT*)A.out;
-  for (int64_t item = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; item < items;
-       item += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t t = item / A.nchunks;
-    const int q = (int)(item - t * A.nchunks);
-    const int c0 = q * V;
-    const int valid = min(V, C - c0);
-    const int64_t base = t * n * C + c0;
-    float agg[V];
+  for (int64_t item0 = (int64_t)blockIdx.x * (kResThreads * K) + threadIdx.x; item0 < items;
+       item0 += (int64_t)gridDim.x * (kResThreads * K)) {
+    int64_t base[K], to[K];
+    bool in[K];
+    float agg[K][V];
 #pragma unroll
-    for (int v = 0; v < V; ++v) agg[v] = 0.0f;
-    for (int i0 = 0; i0 < n; i0 += G) {
-      Vec<XT, V> xr[G], rr[G];
+    for (int k = 0; k < K; ++k) {
+      const int64_t item = item0 + k * kResThreads;
+      in[k] = item < items;
+      const int64_t t = items <= UINT32_MAX ? (int64_t)((uint32_t)item / (uint32_t)A.nchunks) : item / A.nchunks;
+      const int c0 = (int)(item - t * A.nchunks) * V;
+      base[k] = t * n * C + c0;
+      to[k] = t * C + c0;
 #pragma unroll
-      for (int g = 0; g < G; ++g) {
-        if (i0 + g < n) {
-          load_c<XT>(xr[g], X + base + (int64_t)(i0 + g) * C, A.vec, valid);
-          load_c<XT>(rr[g], R + base + (int64_t)(i0 + g) * C, A.vec, valid);
-        }
-      }
-#pragma unroll
-      for (int g = 0; g < G; ++g) {
-        if (i0 + g < n) {
-          const float a = s_a[i0 + g];
-          float o[V];
-#pragma unroll
-          for (int v = 0; v < V; ++v) {
-            o[v] = xr[g].get(v) + rr[g].get(v);
-            agg[v] = fmaf(o[v], a, agg[v]);
-          }
-          store_c<OT>(O + base + (int64_t)(i0 + g) * C, o, A.vec, valid);
-        }
-      }
+      for (int v = 0; v < V; ++v) agg[k][v] = 0.0f;
     }
-    store_c<float>(A.y_agg + t * C + c0, agg, A.vec, valid);
+    for (int i0 = 0; i0 < n; i0 += G) {
+      Vec<XT, V> xr[K][G], rr[K][G];
+#pragma unroll
+      for (int k = 0; k < K; ++k)
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+          if (in[k] && i0 + g < n) {
+            xr[k][g].template load<NT>(X + base[k] + (int64_t)(i0 + g) * C);
+            rr[k][g].template load<NT>(R + base[k] + (int64_t)(i0 + g) * C);
+          }
+#pragma unroll
+      for (int k = 0; k < K; ++k)
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+          if (in[k] && i0 + g < n) {
+            const float a = s_a[i0 + g];
+            float o[V];
+#pragma unroll
+            for (int v = 0; v < V; ++v) {
+              o[v] = xr[k][g].get(v) + rr[k][g].get(v);
+              agg[k][v] = fmaf(o[v], a, agg[k][v]);
+            }
+            res_store<OT, V, NT>(O + base[k] + (int64_t)(i0 + g) * C, o);
+          }
+    }
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+      if (in[k]) res_store<float, V, NT>(A.y_agg + to[k], agg[k]);
   }
 }
 
@@ -212,8 +255,8 @@ int res_group(int n) { return n <= 4 ? 4 : 8; }
 constexpr int kResBwdGroup = 4;
 
 // One item per thread (the grid-stride loop then runs once) measured best on
-// MI355X: 646 us at 32768 x 4 x 4096 bf16 (72.7% of 8 TB/s) against 675-700 us
-// for persistent grids of 2-32 blocks per CU.  MHC_RES_GRID > 0 caps the grid
+// MI355X: 4% faster at 32768 x 4 x 4096 bf16 than the best of the persistent
+// grids of 2-32 blocks per CU.  MHC_RES_GRID > 0 caps the grid
 // at that many blocks per CU (tuning override).
 int64_t res_fwd_grid(int64_t items, int cus) {
   const int64_t g = ceil_div(items, kResThreads);
@@ -228,11 +271,11 @@ int64_t res_bwd_grid(int64_t T, int n, int C, int cus) {
   return std::max<int64_t>(1, std::min<int64_t>(g, (int64_t)cus * 8 / groups + 1));
 }
 
-bool res_vec_ok(int C, std::initializer_list<std::pair<const void*, int>> ptrs) {
-  if (C % kResV != 0) return false;
+bool res_vec_ok(int C, int V, std::initializer_list<std::pair<const void*, int>> ptrs) {
+  if (C % V != 0) return false;
   for (auto& pr : ptrs) {
     if (pr.first == nullptr) continue;
-    const int al = std::min(16, kResV * pr.second);
+    const int al = std::min(16, V * pr.second);
     if (!aligned(pr.first, al)) return false;
   }
   return true;
@@ -272,10 +315,14 @@ extern "C" int mhc_residual_add_agg_fwd(const void* x, const void* res, int dtyp
   ResArgs A{};
   A.x = x; A.res = res; A.out = out; A.y_agg = y_agg; A.hpre = h_pre; A.T = T; A.n = n; A.C = C;
   A.h_mode = h_mode;
-  A.nchunks = (int)ceil_div(C, kResV);
-  A.vec = res_vec_ok(C, {{x, dtype_bytes(dtype)}, {res, dtype_bytes(dtype)}, {out, dtype_bytes(out_dtype)},
-                         {y_agg, 4}});
-  const int64_t blocks = res_fwd_grid(T * A.nchunks, device_cu_count());
+  const int bx = dtype_bytes(dtype), bo = dtype_bytes(out_dtype);
+  auto fits = [&](int v) { return res_vec_ok(C, v, {{x, bx}, {res, bx}, {out, bo}, {y_agg, 4}}); };
+  const int V = bx == 2 && bo == 2 && fits(8) ? 8 : fits(4) ? 4 : 1;
+  // Non-temporal for rows of whole 128-byte lines; other rows share lines with their neighbours (3000 x 16 x 1100 fp16
+  // to fp32: 92 us cached, 95 with the hint).
+  const bool nt = V > 1 && (int64_t)C * bx % 128 == 0 && (int64_t)C * bo % 128 == 0;
+  A.nchunks = C / V;
+  const int64_t blocks = res_fwd_grid(ceil_div(T * A.nchunks, V > 1 ? 1 : res_group(n) > 4 ? 2 : 4), device_cu_count());
   hipStream_t s = (hipStream_t)stream;
   return res_by_group(n, [&](auto gc) {
     constexpr int G = decltype(gc)::value;
@@ -283,10 +330,22 @@ extern "C" int mhc_residual_add_agg_fwd(const void* x, const void* res, int dtyp
       using XT = std::remove_pointer_t<decltype(xp)>;
       return res_by_dtype(out_dtype, [&](auto* op) {
         using OT = std::remove_pointer_t<decltype(op)>;
-        hipLaunchKernelGGL((residual_add_agg_kernel<G, XT, OT>), dim3((unsigned)blocks), dim3(kResThreads),
-                           0, s, A);
-        MHC_CHECK_LAUNCH("residual_add_agg_kernel");
-        return MHC_OK;
+        auto go = [&](auto vc, auto ntc) {
+          hipLaunchKernelGGL((residual_add_agg_kernel<G, XT, OT, decltype(vc)::value, decltype(ntc)::value>),
+                             dim3((unsigned)blocks), dim3(kResThreads), 0, s, A);
+          MHC_CHECK_LAUNCH("residual_add_agg_kernel");
+          return (int)MHC_OK;
+        };
+        using std::integral_constant;
+        if constexpr (sizeof(XT) == 2 && sizeof(OT) == 2) {
+          if (V == 8) {
+            return nt ? go(integral_constant<int, 8>{}, std::true_type{}) : go(integral_constant<int, 8>{}, std::false_type{});
+          }
+        }
+        if (V == 4) {
+          return nt ? go(integral_constant<int, 4>{}, std::true_type{}) : go(integral_constant<int, 4>{}, std::false_type{});
+        }
+        return go(integral_constant<int, 1>{}, std::false_type{});
       });
     });
   });
@@ -333,7 +392,7 @@ extern "C" int mhc_residual_add_agg_bwd(const void* x, const void* res, int dtyp
   A.part = dh_pre ? (float*)workspace : nullptr;
   A.T = T; A.n = n; A.C = C; A.nchunks = (int)ceil_div(C, kResV); A.h_mode = h_mode; A.P = P;
   const int gdt = dout ? dout_dtype : dtype;
-  A.vec = res_vec_ok(C, {{x, dtype_bytes(dtype)}, {res, dtype_bytes(dtype)}, {dout, dtype_bytes(gdt)},
+  A.vec = res_vec_ok(C, kResV, {{x, dtype_bytes(dtype)}, {res, dtype_bytes(dtype)}, {dout, dtype_bytes(gdt)},
                          {dy_agg, 4}, {dx, dtype_bytes(dtype)}, {dres, dtype_bytes(dtype)}});
   hipStream_t s = (hipStream_t)stream;
   const int groups = (int)ceil_div(n, kResBwdGroup);

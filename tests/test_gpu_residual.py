@@ -42,6 +42,30 @@ def test_forward_matches_oracle(B, n, C, dt):
     assert rel_err(np_of(y), ry) < 1e-5
 
 
+@pytest.mark.parametrize("B,n,C", [(3, 4, 4), (41, 5, 100), (70, 3, 36), (37, 9, 61), (300, 4, 7), (33, 8, 96), (1100, 2, 1)])
+@pytest.mark.parametrize("xdt,odt", [("f32", "f32"), ("bf16", "f32"), ("f16", "f16"), ("f32", "bf16")])
+@pytest.mark.parametrize("shift", [0, 1])
+@pytest.mark.parametrize("grid", [None, 1])
+def test_forward_widths(B, n, C, xdt, odt, shift, grid, knobs):
+    """Rows taken eight, four and one channel at a time, on one block per CU too; operands that start `shift` elements
+    into an allocation (no vector of theirs is aligned) give bitwise the same results."""
+    if grid is not None:
+        knobs("MHC_RES_GRID", grid)
+    x, res, h = _inputs(B, n, C, xdt, 17 + B + n + C)
+
+    def moved(a):
+        t = torch.empty(a.numel() + 1, dtype=a.dtype, device="cuda")[shift:shift + a.numel()].view(a.shape)
+        return t.copy_(a)
+
+    args = dev_tensor(x, xdt), dev_tensor(res, xdt)
+    out, y = ops.residual_add_agg_hip(*map(moved, args), dev_tensor(h), output_dtype=TORCH_DT[odt])
+    again = ops.residual_add_agg_hip(*args, dev_tensor(h), output_dtype=TORCH_DT[odt])
+    assert torch.equal(out, again[0]) and torch.equal(y, again[1])
+    ro, ry = O.residual_add_agg(x, res, h, dtype=np.float32)
+    assert np.array_equal(np_of(out), to_dtype_np(ro, odt).astype(np.float64))  # one fp32 add, rounded once
+    assert rel_err(np_of(y), O.residual_add_agg(x, res, h)[1]) < 1e-5
+
+
 @pytest.mark.parametrize("xdt", ["f32", "bf16", "f16"])
 @pytest.mark.parametrize("odt", ["bf16", "f16"])
 def test_half_output_is_rounded_sum(xdt, odt):
