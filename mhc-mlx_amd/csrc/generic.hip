@@ -3,8 +3,10 @@
 // A persistent workgroup walks tokens; threads own channels, keep a
 // channel's n values in registers and mix them against rows of M broadcast
 // from LDS; parameter-gradient sums are 4 x 4 outer-product blocks, one per
-// wavefront.  The kernels in fused_fwd.hip / fused_bwd.hip / stream_mix.hip
-// cover n <= 16.
+// wavefront.  They are the last resort, for what the matrix-core kernels
+// (mfma32.hip, lf32_*, mix32.hip, mxf32_*) decline: tokens past their LDS or
+// their 32-bit offsets.  The kernels in fused_fwd.hip / fused_bwd.hip /
+// stream_mix.hip cover n <= 16.
 #include <type_traits>
 
 #include "mhc_device.hpp"

@@ -44,7 +44,7 @@ namespace mhc {
 namespace {
 
 template <typename XT, typename OT, int NB, int SPW, int MODE, bool PT>
-__global__ __launch_bounds__(64 * kLfMaxWaves) void lf32_fwd_kernel(GenArgs A) {
+__global__ __launch_bounds__(64 * kLfMaxWaves) void lf32_fwd_kernel(GenFwdArgs A) {
   constexpr bool VEC = MODE != kLfElem;
   constexpr int NK = 4 * NB;
   constexpr int NJ = SPW > 0 ? SPW : 1;
@@ -320,7 +320,7 @@ int lf_fwd_launch(const GenArgs& A, int waves, hipStream_t s) {
   int64_t blocks = (int64_t)device_cu_count() * (per_cu > 0 ? per_cu : occ);
   blocks = std::max<int64_t>(1, std::min<int64_t>(A.T, blocks));
   hipLaunchKernelGGL((lf32_fwd_kernel<XT, OT, NB, SPW, MODE, PT>), dim3((unsigned)blocks), dim3(waves * 64), smem, s,
-                     A);
+                     GenFwdArgs(A));
   MHC_CHECK_LAUNCH("lf32_fwd_kernel");
   return MHC_OK;
 }

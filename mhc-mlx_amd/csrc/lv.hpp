@@ -135,7 +135,8 @@ MHC_DEV void lv_store(__amdgpu_buffer_rsrc_t rs, const LvAt<MODE>& at, uint32_t 
 template <int NMAX>
 struct LvParams {
   float M[NMAX * NMAX], a[NMAX], p[NMAX];
-  MHC_DEV void load(const GenArgs& A, int64_t t, int lane) {
+  template <typename Args>
+  MHC_DEV void load(const Args& A, int64_t t, int lane) {
     const int n = A.n;
     typedef const float __attribute__((address_space(4))) cfloat;
     cfloat* m = (cfloat*)(uintptr_t)(A.M + t * A.M_ts);
@@ -196,7 +197,7 @@ MHC_DEV float lv_sum(float v) {
 // Forward
 // ---------------------------------------------------------------------------
 template <int NMAX, typename XT, typename OT, int MODE, int SPW, int G, bool PT>
-__global__ __launch_bounds__(64 * kLvMaxWaves) void lv_fwd_kernel(GenArgs A, int wpt) {
+__global__ __launch_bounds__(64 * kLvMaxWaves) void lv_fwd_kernel(GenFwdArgs A, int wpt) {
   constexpr int V = lv_width(MODE);
   constexpr int NJ = SPW > 0 ? SPW : 1;
   static_assert(G == 64 || (!PT && SPW == 1), "several tokens per wave: layer-wide, one chunk");
@@ -775,8 +776,8 @@ int lv_fwd_typed(const GenArgs& A, hipStream_t s) {
           const int per_cu = knob(kKnobFwdGrid, 0);
           int64_t blocks = (int64_t)device_cu_count() * (per_cu > 0 ? per_cu : occ);
           blocks = std::max<int64_t>(1, std::min(blocks, ceil_div(A.T, lv_tokens(wpt, G))));
-          hipLaunchKernelGGL((lv_fwd_kernel<NM, XT, OT, MODE, SPW, G, PT>), dim3((unsigned)blocks), dim3(tpb), 0, s, A,
-                             wpt);
+          hipLaunchKernelGGL((lv_fwd_kernel<NM, XT, OT, MODE, SPW, G, PT>), dim3((unsigned)blocks), dim3(tpb), 0, s,
+                             GenFwdArgs(A), wpt);
           MHC_CHECK_LAUNCH("lv_fwd_kernel");
           return (int)MHC_OK;
         };
