@@ -24,7 +24,7 @@ struct FwdCfg {
 };
 
 // Register-tiled kernels exist for NMAX in {4, 8, 16}; 0 selects the
-// runtime-n kernels of generic.hip (16 < n <= 64).
+// kernels for 16 < n <= 64 (matrix cores first, generic.hip for what those decline).
 inline int nmax_for(int n) { return n <= 4 ? 4 : (n <= 8 ? 8 : (n <= 16 ? 16 : 0)); }
 inline int fwd_vec_width(int nmax) { return nmax <= 8 ? 8 : 64 / nmax; }
 inline int bwd_vec_width(int nmax) { return nmax <= 4 ? 8 : (nmax == 8 ? 4 : (nmax == 16 ? 2 : 1)); }
