@@ -568,7 +568,8 @@ __global__ __launch_bounds__(64 * kLvMaxWaves) void lv_bwd_kernel(GenArgs A, int
 #pragma unroll
           for (int k = 0; k < Vec<GT, V>::kWords; ++k) g[j][i].w[k] = lf_opaque(g[j][i].w[k]);
         }
-        give(j, ro, dw[j]);
+        // (a place past the last token stays out: its rows are zero, and with eps = 0 its inv is infinite and kf NaN)
+        if (G == 64 || (uint32_t)W.sub < nt) give(j, ro, dw[j]);
       }
     } else {
       for (int s = W.part; s < S; s += wpt) {

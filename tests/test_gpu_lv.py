@@ -83,3 +83,39 @@ def test_lv_matches_the_tile_kernel(n, C, knobs):
         for a, b in zip(res[0], other):
             assert rel_err(np_of(a), np_of(b)) < 1e-5
     assert not all(torch.equal(a, b) for a, b in zip(res[0][1:], res[2][1:]))
+
+
+@pytest.mark.parametrize("T,n,C", [(37, 4, 64), (1, 2, 33), (18, 8, 100), (5, 3, 128), (37, 4, 200), (3, 4, 777)])
+@pytest.mark.parametrize("xdt,odt", [("f32", "f32"), ("bf16", "bf16"), ("f16", "f32")])
+@pytest.mark.parametrize("eps", [0.0, 1e-30])
+def test_lv_without_eps(T, n, C, xdt, odt, eps, knobs):
+    """eps = 0, and an eps whose inv^3 overflows: a wave's token places past the last token have no RMS norm, and nothing
+    of them may reach the parameter gradients (16, 32 and 64 lanes per token; counts that leave places empty)."""
+    g = rng(9900 + T + C)
+    x, dout = to_dtype_np(g.standard_normal((T, n, C)), xdt), to_dtype_np(g.standard_normal((T, n, C)), odt)
+    ps = params(g, n, C)
+    xt = dev_tensor(x, xdt).requires_grad_(True)
+    pt = [dev_tensor(v).requires_grad_(True) for v in ps]
+    out = ops.mhc_layer_forward(xt, *pt, sinkhorn_iters=20, eps=eps, output_dtype=None if odt == "f32" else xt.dtype)
+    got = [out.detach(), *torch.autograd.grad(out, [xt, *pt], dev_tensor(dout, odt))]
+    refs = [O.mhc_forward_reference(x, *ps, sinkhorn_iters=20, eps=eps),
+            *O.mhc_backward_reference(x, *ps, dout, sinkhorn_iters=20, eps=eps)]
+    for name, a, r in zip(("out", "dx", "dH_pre", "dH_post", "dH_res", "d_w"), got, refs):
+        tol = TOL[odt] if name == "out" else (TOL[xdt] if name == "dx" else GRAD_TOL)
+        assert rel_err(np_of(a), r, floor=1e-3) < tol, (name, rel_err(np_of(a), r, floor=1e-3))
+
+
+@pytest.mark.parametrize("n,C", [(4, 64), (3, 33), (8, 100), (4, 300), (6, 777)])
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_lv_non_finite_stays_in_its_token(n, C, bad):
+    """Several tokens share a wave: an infinity or a NaN of one reaches that token's rows and no other's."""
+    T, t = 11, 5
+    g = rng(9950 + C)
+    x = dev_tensor(g.standard_normal((T, n, C)))
+    x[t, n - 1, C // 2] = bad
+    xt = x.requires_grad_(True)
+    out = ops.mhc_layer_forward(xt, *(dev_tensor(v) for v in params(g, n, C)), eps=EPS)
+    dx, = torch.autograd.grad(out, xt, dev_tensor(g.standard_normal((T, n, C))))
+    others = [k for k in range(T) if k != t]
+    assert torch.isfinite(out[others]).all() and torch.isfinite(dx[others]).all()
+    assert not torch.isfinite(out[t, :, C // 2]).any() and torch.isnan(dx[t]).any()
