@@ -113,6 +113,16 @@ def _binding():
     return _BINDING
 
 
+def _use_binding() -> bool:
+    """Whether a call may go through the binding's C++ Functions.
+
+    Not under a kernel timer, which times the Python Functions' launches, and not while torch.jit.trace
+    records: it keeps a Python Function as a node and runs it again on replay, but of a C++ one only the
+    allocations, so that a replay would return memory that nothing has written.
+    """
+    return profiling._active is None and not torch._C._is_tracing()
+
+
 def _ws(nbytes: int, dev) -> torch.Tensor | None:
     if nbytes <= 0:
         return None
@@ -764,7 +774,7 @@ def post_combine(x, y_inner, H_pre_raw, H_post_raw, H_res_raw, sinkhorn_iters: i
     if out_dtype not in (torch.float32, x.dtype):
         raise ValueError(f"unsupported output_dtype: {output_dtype}")
     _require_gpu(x, y_inner, H_pre_raw, H_post_raw, H_res_raw)
-    if profiling._active is None and int(H_pre_raw.numel()) == n and int(H_post_raw.numel()) == n:
+    if _use_binding() and int(H_pre_raw.numel()) == n and int(H_post_raw.numel()) == n:
         return _binding().post_combine(x, y_inner, H_pre_raw, H_post_raw, H_res_raw, int(sinkhorn_iters), float(eps),
                                        _DTYPE_CODE[out_dtype])
     return PostCombineFn.apply(x, y_inner, H_pre_raw, H_post_raw, H_res_raw, int(sinkhorn_iters),
@@ -824,7 +834,7 @@ def _stream_scale_check(x, H_pre_raw):
 def stream_scale(x, H_pre_raw):
     """Pre-scale of MHCRewire: [B, n, C] * sigmoid(H_pre_raw)[n]."""
     _stream_scale_check(x, H_pre_raw)
-    if profiling._active is None:
+    if _use_binding():
         return _binding().stream_scale(x, H_pre_raw, False)[0]
     return StreamScaleFn.apply(x, H_pre_raw, False)
 
@@ -833,7 +843,7 @@ def stream_scale_and_pass(x, H_pre_raw):
     """(stream_scale(x, H_pre_raw), x): the second output is x for a second use (MHCRewire's
     post-combine) whose gradient the pre-scale's VJP adds into dx in its own pass."""
     _stream_scale_check(x, H_pre_raw)
-    if profiling._active is None:
+    if _use_binding():
         return tuple(_binding().stream_scale(x, H_pre_raw, True))
     return StreamScaleFn.apply(x, H_pre_raw, True)
 
@@ -927,7 +937,7 @@ def residual_add_agg_hip(x, res, H_pre, threads_per_group=None, output_dtype=Non
     else:
         raise ValueError(f"unsupported output_dtype: {output_dtype}")
     _require_gpu(x, res, H_pre)
-    if (profiling._active is None and x.dtype == res.dtype and not _needs_grad(x, res, H_pre)
+    if (_use_binding() and x.dtype == res.dtype and not _needs_grad(x, res, H_pre)
             and torch.autograd.forward_ad._current_level < 0):  # (forward mode is refused by the Function)
         return _binding().residual_add_agg_nograd(x, res, H_pre, _DTYPE_CODE[out_dtype])
     return ResidualAddAggFn.apply(x, res, H_pre, out_dtype)

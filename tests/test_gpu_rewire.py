@@ -466,3 +466,27 @@ def test_rewire_binding_matches_the_python_functions(n, xdt, ydt, pdt):
         b = run()
     for u, v in zip(a, b):
         assert u.dtype == v.dtype and u.shape == v.shape and torch.equal(u, v)
+
+
+@pytest.mark.parametrize("grad", [False, True])
+def test_traced_calls_run_the_kernels_again(grad):
+    """torch.jit.trace of MHCRewire and of residual_add_agg: a replay on other inputs gives their results and gradients."""
+    from mhc_mlx_amd import residual_add_agg
+
+    torch.manual_seed(0)
+    dims, n, T = 96, 4, 6
+    m = MHCRewire(torch.nn.Linear(dims, dims, device="cuda"), dims, n=n, device="cuda")
+    x, other = (torch.randn(T, dims, device="cuda") for _ in range(2))
+    r, h = torch.randn(T, n, dims // n, device="cuda"), torch.rand(n, device="cuda")
+    with torch.set_grad_enabled(grad):
+        rewire = torch.jit.trace(m, (x,), check_trace=False)
+        add = torch.jit.trace(residual_add_agg, (x.view(T, n, -1), r, h), check_trace=False)
+        xs = [other.clone().requires_grad_(grad) for _ in range(2)]
+        got, want = rewire(xs[0]), m(xs[1])
+        assert torch.equal(got, want)
+        for u, v in zip(add(other.view(T, n, -1), r, h), residual_add_agg(other.view(T, n, -1), r, h)):
+            assert torch.equal(u, v)
+    if grad:
+        for u, v in zip(torch.autograd.grad(got.sum(), [xs[0], m.mhc.H_res_raw]),
+                        torch.autograd.grad(want.sum(), [xs[1], m.mhc.H_res_raw])):
+            assert torch.equal(u, v)
