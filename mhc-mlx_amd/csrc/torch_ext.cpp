@@ -17,6 +17,7 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Dtype.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 
 #include "mhc_hip.h"
 
@@ -397,8 +398,9 @@ bool env_is_one(const char* name) {
 // getenv, which sees os.environ's changes, as the reference reads its switch
 // per call, layer.py:176) or when the call is not one this path takes (x not
 // [B, n, C] for the layer's n and C, tensors off x's GPU, n > 64, a dtype the
-// kernels do not read), so that the module's general path decides and raises
-// the reference's errors.  Otherwise the output: the kernel writes
+// kernels do not read; or torch.jit.trace is recording, which would keep only
+// this call's allocations), so that the module's general path decides and
+// raises the reference's errors.  Otherwise the output: the kernel writes
 // return_dtype directly when it is x's half type (layer.py:361-364), else fp32
 // cast to return_dtype; the autograd node is recorded when grad mode is on and
 // x or a parameter requires a gradient.
@@ -406,6 +408,7 @@ at::Tensor module_forward(const at::Tensor& x, const at::Tensor& hpre, const at:
                           const at::Tensor& hres, const at::Tensor& w, int64_t n, int64_t C, int64_t iters,
                           double eps, c10::optional<at::ScalarType> return_dtype) {
   if (env_is_one("MHC_MLX_DISABLE_METAL") || env_is_one("MHC_HIP_DISABLE")) return at::Tensor();
+  if (torch::jit::tracer::isTracing()) return at::Tensor();
   if (n < 1 || n > MHC_MAX_N || x.dim() != 3 || x.size(1) != n || x.size(2) != C || !x.is_cuda()) return at::Tensor();
   const at::ScalarType xt = x.scalar_type();
   if (xt != at::kFloat && xt != at::kBFloat16 && xt != at::kHalf) return at::Tensor();

@@ -343,7 +343,7 @@ class MHCLayer(nn.Module):
         dtypes, allocates the output and, when a gradient is needed, records the C++ autograd node whose
         backward runs the library's VJP.  At small batch the layer's latency is mostly this host code.
         It returns None whenever the general path below has something to decide (a disable switch,
-        use_metal off, a shape error, tensors off the GPU, n > 64, a kernel timer, a library error).
+        use_metal off, a shape error, tensors off the GPU, n > 64, a kernel timer, a trace, a library error).
         """
         if profiling._active is None:
             try:

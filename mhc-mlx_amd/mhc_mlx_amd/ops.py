@@ -429,11 +429,11 @@ def layer_apply(x, hpre, hpost, hres, w, iters: int, eps: float, out_dtype):
     """MHCLayer's forward with autograd through the torch binding, with the fewest host steps.
 
     Layer-wide parameters with the layer's shapes; x on a GPU in fp32/bf16/fp16.  Returns None when the
-    dtype is not one the library takes or a kernel timer is active (the caller takes the general path);
+    dtype is not one the library takes or the binding may not be used (the caller takes the general path);
     raises ValueError for tensors on another device and RuntimeError on a library error.  n > 16 records
     the Sinkhorn VJP state, as mhc_layer_forward does.
     """
-    if x.dtype not in _DTYPE_CODE or not x.is_cuda or profiling._active is not None:
+    if x.dtype not in _DTYPE_CODE or not x.is_cuda or not _use_binding():
         return None
     return _binding().layer_apply(x, hpre, hpost, hres, w, iters, eps, _DTYPE_CODE[out_dtype], False,
                                   x.shape[1] > 16)
@@ -449,7 +449,7 @@ def layer_forward_nograd(x, hpre, hpost, hres, w, iters: int, eps: float, out_dt
     on another device and RuntimeError on a library error.  out_dtype: torch.float32, or x's dtype
     when that is 16-bit.
     """
-    if x.dtype not in _DTYPE_CODE or not x.is_cuda or profiling._active is not None:
+    if x.dtype not in _DTYPE_CODE or not x.is_cuda or not _use_binding():
         return None
     return _binding().layer_forward_nograd(x, hpre, hpost, hres, w, iters, eps, _DTYPE_CODE[out_dtype], False)
 
@@ -612,10 +612,11 @@ def mhc_layer_forward(x, H_pre_raw, H_post_raw, H_res_raw, rms_weight, sinkhorn_
     _fused_shapes(x, H_res_raw, H_pre_raw, H_post_raw, rms_weight)
     out_dtype = _normalize_output_dtype(output_dtype, x.dtype)
     _require_gpu(x, H_pre_raw, H_post_raw, H_res_raw, rms_weight)
-    if not _needs_grad(x, H_pre_raw, H_post_raw, H_res_raw, rms_weight):
+    # (while a trace is recorded the Function runs whatever the gradients: the trace keeps it as a node)
+    if not _needs_grad(x, H_pre_raw, H_post_raw, H_res_raw, rms_weight) and not torch._C._is_tracing():
         return _layer_fwd(x, H_pre_raw, H_post_raw, H_res_raw, rms_weight, int(sinkhorn_iters), float(eps),
                           out_dtype, False)[0]
-    if profiling._active is None:
+    if _use_binding():
         # the same Function in C++ (backward without Python); n > 16 records the Sinkhorn state
         return _binding().layer_apply(x, H_pre_raw, H_post_raw, H_res_raw, rms_weight, int(sinkhorn_iters),
                                       float(eps), _DTYPE_CODE[out_dtype], False, int(x.shape[1]) > 16)
@@ -631,7 +632,7 @@ def mhc_layer_forward_dynamic(x, H_pre_raw, H_post_raw, H_res_raw, rms_weight, s
     _fused_shapes(x, H_res_raw, H_pre_raw, H_post_raw, rms_weight)
     out_dtype = _normalize_output_dtype(output_dtype, x.dtype)
     _require_gpu(x, H_pre_raw, H_post_raw, H_res_raw, rms_weight)
-    if profiling._active is None and _needs_grad(x, H_pre_raw, H_post_raw, H_res_raw, rms_weight):
+    if _use_binding() and _needs_grad(x, H_pre_raw, H_post_raw, H_res_raw, rms_weight):
         return _binding().layer_apply(x, H_pre_raw, H_post_raw, H_res_raw, rms_weight, int(sinkhorn_iters),
                                       float(eps), _DTYPE_CODE[out_dtype], True, True)
     return MHCLayerFn.apply(x, H_pre_raw, H_post_raw, H_res_raw, rms_weight, int(sinkhorn_iters),

@@ -211,3 +211,24 @@ def test_nograd_n_above_64_takes_the_reference_path(grad_mode, fast_calls):
     ref = O.mhc_forward_reference(np_of(x), hpre, hpost, hres, w, sinkhorn_iters=20, eps=1e-6)
     assert out.dtype == torch.float32 and out.is_cuda
     assert rel_err(np_of(out), ref) < 1e-5
+
+
+@pytest.mark.parametrize("n", [4, 20])
+@pytest.mark.parametrize("grad", [False, True])
+def test_traced_layer_runs_the_kernels_again(n, grad):
+    """torch.jit.trace of MHCLayer.forward and forward_dynamic: a replay on other inputs gives their results and
+    gradients."""
+    T, C = 5, 24
+    g = rng(190 + n)
+    layer, _ = _layer(n, C, g)
+    x, other, dout = (dev_tensor(g.standard_normal((T, n, C))) for _ in range(3))
+    H = [dev_tensor(v) for v in params(g, n, C, per_token_B=T)[:3]]
+    with torch.set_grad_enabled(grad):
+        plain = torch.jit.trace(layer, (x,), check_trace=False)
+        dynamic = torch.jit.trace_module(layer, {"forward_dynamic": (x, *H)}, check_trace=False).forward_dynamic
+        for traced, call, args in ((plain, layer, ()), (dynamic, layer.forward_dynamic, H)):
+            xs = [other.clone().requires_grad_(grad) for _ in range(2)]
+            got, want = traced(xs[0], *args), call(xs[1], *args)
+            assert torch.equal(got, want)
+            if grad:
+                assert torch.equal(torch.autograd.grad(got, xs[0], dout)[0], torch.autograd.grad(want, xs[1], dout)[0])
