@@ -243,9 +243,10 @@ __global__ __launch_bounds__(64 * kLvMaxWaves) void lv_fwd_kernel(GenFwdArgs A, 
       float o[V];
 #pragma unroll
       for (int v = 0; v < V; ++v) {
-        o[v] = P.p[i] * yn[v];
+        o[v] = 0.0f;
 #pragma unroll
         for (int k = 0; k < NMAX; ++k) o[v] = fmaf(P.M[i * NMAX + k], x[j][k].get(v), o[v]);
+        o[v] = fmaf(P.p[i], yn[v], o[v]);  // last: the largest term, and each sum is rounded at its own size
       }
       lv_store<OT, MODE>(ro, at[j].fresh(), subo + (i < n ? (uint32_t)i * rowo : kLvNoRow), o);
     }
@@ -468,10 +469,10 @@ __global__ __launch_bounds__(64 * kLvMaxWaves) void lv_bwd_kernel(GenArgs A, int
       if constexpr (!kRows) {
 #pragma unroll
         for (int k = 0; k < NMAX; ++k) {
-          float s = P.a[k] * dy[v];
+          float s = 0.0f;
 #pragma unroll
           for (int i = 0; i < NMAX; ++i) s = fmaf(P.M[i * NMAX + k], gs[i], s);
-          o[k][v] = s;
+          o[k][v] = fmaf(P.a[k], dy[v], s);
         }
       }
 #pragma unroll
@@ -498,9 +499,10 @@ __global__ __launch_bounds__(64 * kLvMaxWaves) void lv_bwd_kernel(GenArgs A, int
         if constexpr (NMAX > 4) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int v = 0; v < V; ++v) {
-          o[0][v] = P.a[k] * dy[v];
+          o[0][v] = 0.0f;
 #pragma unroll
           for (int i = 0; i < NMAX; ++i) o[0][v] = fmaf(P.M[i * NMAX + k], g[j][i].get(v), o[0][v]);
+          o[0][v] = fmaf(P.a[k], dy[v], o[0][v]);
         }
       }
       lv_store<XT, MODE>(ro, at[j].fresh(), subx + (k < n ? (uint32_t)k * rowx : kLvNoRow), o[kRows ? 0 : k]);

@@ -119,3 +119,39 @@ def test_lv_non_finite_stays_in_its_token(n, C, bad):
     others = [k for k in range(T) if k != t]
     assert torch.isfinite(out[others]).all() and torch.isfinite(dx[others]).all()
     assert not torch.isfinite(out[t, :, C // 2]).any() and torch.isnan(dx[t]).any()
+
+
+def _fma(a, b, c):
+    return (a.astype(np.float64) * b + c).astype(np.float32)
+
+
+@pytest.mark.parametrize("T,n,C", [(400, 8, 100), (130, 7, 1001), (130, 8, 2001), (300, 8, 252)])
+def test_lv_rounds_no_more_than_its_sums_need(T, n, C):
+    """fp32 out and dx are no further from float64 than the same sums in numpy's fp32 with the mix first and the
+    (larger) RMS term added last; the RMS term first rounds every product against it, 1.3 times the error.  The bound's 15%
+    covers the order of the RMS sums, whose error a token's channels share."""
+    g = rng(9990 + n)
+    x, dout = (g.standard_normal((T, n, C)).astype(np.float32) for _ in range(2))
+    M = O.mixing_matrix_from_logits(g.standard_normal((n, n)), 20, EPS).astype(np.float32)
+    a, p = g.uniform(size=n).astype(np.float32), (2 * g.uniform(size=n)).astype(np.float32)
+    w = (1 + 0.02 * g.standard_normal(C)).astype(np.float32)
+    ts = [dev_tensor(v).requires_grad_(True) for v in (x, M, a, p, w)]
+    out = ops.mhc_forward_fused_hip_autograd(*ts, eps=EPS)
+    dx, = torch.autograd.grad(out, ts[0], dev_tensor(dout))
+
+    y, d = np.zeros((T, C), np.float32), np.zeros((T, C), np.float32)
+    for i in range(n):
+        y, d = _fma(a[i], x[:, i], y), _fma(p[i], dout[:, i], d)
+    ss = (y.astype(np.float64) ** 2).sum(-1, keepdims=True).astype(np.float32)
+    inv = np.float32(1) / np.sqrt(ss / np.float32(C) + np.float32(EPS))
+    kf = (inv * inv * inv / np.float32(C)) * (d.astype(np.float64) * y * w).sum(-1, keepdims=True).astype(np.float32)
+    yn, dy = y * inv * w, d * inv * w - kf * y
+    exact = (O.mhc_forward_fused_reference(x, M, a, p, w, eps=EPS), O.mhc_fused_backward(x, M, a, p, w, dout, eps=EPS)[0])
+    for got, ref, mat, rows, last, scale in ((np_of(out), exact[0], M, x, yn, p), (np_of(dx), exact[1], M.T, dout, dy, a)):
+        own = np.empty_like(x)
+        for i in range(n):
+            s = np.zeros((T, C), np.float32)
+            for k in range(n):
+                s = _fma(mat[i, k], rows[:, k], s)
+            own[:, i] = _fma(scale[i], last, s)
+        assert np.linalg.norm(got - ref) < 1.15 * np.linalg.norm(own - ref), np.linalg.norm(got - ref) / np.linalg.norm(own - ref)
