@@ -182,15 +182,20 @@ __global__ __launch_bounds__(64 * kMxfWaves) void mxf_fwd_kernel(MxfArgs A) {
 #pragma unroll
       for (int I = 0; I < NB; ++I)
 #pragma unroll
-        for (int v = 0; v < 4; ++v)
-#pragma unroll
-          for (int k = 0; k < 4; ++k) d[I][v][k] = p[I][k] * y[I][k].get(v);
+        for (int v = 0; v < 4; ++v) d[I][v] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
       for (int m = 0; m < NK; ++m)
 #pragma unroll
         for (int v = 0; v < 4; ++v)
 #pragma unroll
           for (int I = 0; I < NB; ++I) d[I][v] = lf_mfma(am[I][m], x[m].get(v), d[I][v]);
+      // y joins last: begun with it, every product of the mix would be rounded against this larger term
+#pragma unroll
+      for (int I = 0; I < NB; ++I)
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+#pragma unroll
+          for (int k = 0; k < 4; ++k) d[I][v][k] = fmaf(p[I][k], y[I][k].get(v), d[I][v][k]);
       const MxfPos<VEC> now = at;
       const bool more = s + stride < slabs;
       if (more) {

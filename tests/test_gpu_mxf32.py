@@ -87,3 +87,19 @@ def test_mxf32_unaligned_rows():
         res.append([out.detach(), *torch.autograd.grad(out, [xs, ys, *ps], ts[2])])
     for a, b in zip(*res):
         assert rel_err(np_of(a), np_of(b)) < 1e-6
+
+
+@pytest.mark.parametrize("T,n,C", [(300, 12, 100), (2000, 16, 20), (500, 24, 40), (900, 32, 32), (130, 6, 333), (100, 40, 100)])
+def test_mxf32_rounds_no_more_than_its_sums_need(T, n, C):
+    """fp32 out is no further from float64 than the same sum in numpy's fp32 with the (larger) y added last; begun with y,
+    every product is rounded against it, three to five times the error.  The bound's 15% covers the order of the mix."""
+    g = rng(9600 + n)
+    x, y = (g.standard_normal((T, n, C)).astype(np.float32) for _ in range(2))
+    M = (g.uniform(size=(n, n)) / n).astype(np.float32)
+    out = np_of(ops.stream_mix_add_hip(dev_tensor(x), dev_tensor(M), dev_tensor(y)))
+    ref = np.matmul(M.astype(np.float64), x) + y
+    own = np.zeros((T, n, C), np.float32)
+    for k in range(n):
+        own = (M[:, k, None].astype(np.float64) * x[:, None, k] + own).astype(np.float32)
+    own = own + y
+    assert np.linalg.norm(out - ref) < 1.15 * np.linalg.norm(own - ref), np.linalg.norm(out - ref) / np.linalg.norm(own - ref)
