@@ -33,7 +33,7 @@
 //
 // Backward kernel, against the VALU kernels before it: 4096 x 32 x 512 fp32
 // 1355 -> 161 us (5.0 TB/s), 4096 x 16 x 1024 fp32 393 -> 140 us (5.8 TB/s),
-// 2048 x 64 x 512 fp32 4145 -> 298 us (one wave per SIMD: dM alone is 64
+// 2048 x 64 x 512 fp32 4145 -> 318 us (one wave per SIMD: dM alone is 64
 // registers), 1024 x 32 x 4096 fp32 3214 -> 400 us, per token 4096 x 32 x 512
 // fp32 1371 -> 190 us and 2500 x 10 x 4000 fp32 479 us (758 us on one wave a token), 3001 x 16 x 1100 fp16 371 -> 101 us and 20000 x 24 x 100
 // bf16 1989 -> 133 us (16-bit rows: bound by the VALU's conversions and LDS).
@@ -206,26 +206,30 @@ __global__ __launch_bounds__(PT ? 64 * kLfPtWaves : (NB > 2 ? 256 : 64 * kLfMaxW
     }
     issue_fence();
   };
-  // dM and the dot products over the slab in LDS.  The slab's products are summed by themselves first: one chain over all
-  // of a wave's slabs would round every product against the whole sum (dH_res at 30000 x 9 x 400 bf16 1.8e-6 off the
-  // exact sum instead of 0.3e-6).  At n > 48 the row blocks of g go in two passes (four per token), so that these partial sums fit.
-  constexpr int IB = NB > 3 ? (PT ? 1 : 2) : NB;
+  // dM and the dot products over the slab in LDS, one row block of g at a time (so that the partial sums are few).  A
+  // slab's products are summed in four chains of 16, and only their sum joins the wave's: one chain over all of a wave's
+  // slabs would round every product against the whole sum (dH_res at 30000 x 9 x 400 bf16 1.8e-6 off the exact sum), one
+  // over a slab against the slab's (dM at 130 x 64 x 512 fp32 1.7e-7 off float64, here 1.2e-7, on the VALU kernel 1.1e-7;
+  // at n = 32, with two chains, 1.8e-7, 1.4e-7 and 1.2e-7).  Prefetched slabs leave registers for two chains of 32, with
+  // SPW = 1 at n <= 16 for one, added at half a slab and at its end (a second one would cost a wave per SIMD), and three
+  // slabs of mixed types for the one of 64 (C > 1024, where the VALU kernel's dM is 2.7e-7 off).  Against one chain:
+  // 4096 x 32 x 512 fp32 149 -> 151 us, 2048 x 64 x 512 299 -> 318, 2048 x 48 x 512 172 -> 181.
+  constexpr bool kHalf = NB == 1 && SPW == 1;
+  constexpr int kChains = SPW == 0 ? 4 : (kHalf || (NB == 1 && SPW == 3 && sizeof(XT) != sizeof(GT)) ? 1 : 2);
   auto sums = [&] {
 #pragma unroll
-    for (int I0 = 0; I0 < NB; I0 += IB) {
-      f32x4 part[IB][NB];
+    for (int I = 0; I < NB; ++I) {
+      f32x4 part[kChains][NB];
 #pragma unroll
-      for (int I = 0; I < IB; ++I)
+      for (int h = 0; h < kChains; ++h)
 #pragma unroll
-        for (int J = 0; J < NB; ++J) part[I][J] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int J = 0; J < NB; ++J) part[h][J] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
         __builtin_amdgcn_sched_barrier(0);  // the four steps' operands at once would take 80-112 registers
         const int c = 16 * k + 4 * q;
-        f32x4 gv[IB], xv[NB];
-#pragma unroll
-        for (int I = 0; I < IB; ++I)
-          gv[I] = *reinterpret_cast<const f32x4*>(sg + (16 * (I0 + I) + r) * kLfPitch + c);
+        const f32x4 gv = *reinterpret_cast<const f32x4*>(sg + (16 * I + r) * kLfPitch + c);
+        f32x4 xv[NB];
 #pragma unroll
         for (int J = 0; J < NB; ++J) xv[J] = *reinterpret_cast<const f32x4*>(sx + (16 * J + r) * kLfPitch + c);
         const f32x4 yv = *reinterpret_cast<const f32x4*>(sc + c);
@@ -234,12 +238,9 @@ __global__ __launch_bounds__(PT ? 64 * kLfPtWaves : (NB > 2 ? 256 : 64 * kLfMaxW
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
 #pragma unroll
-          for (int I = 0; I < IB; ++I)
-#pragma unroll
-            for (int J = 0; J < NB; ++J) part[I][J] = lf_mfma(gv[I][e], xv[J][e], part[I][J]);
-#pragma unroll
-          for (int I = 0; I < IB; ++I) ug[I0 + I] = fmaf(gv[I][e], yw[e], ug[I0 + I]);
-          if (I0 == 0) {
+          for (int J = 0; J < NB; ++J) part[e % kChains][J] = lf_mfma(gv[e], xv[J][e], part[e % kChains][J]);
+          ug[I] = fmaf(gv[e], yw[e], ug[I]);
+          if (I == 0) {
 #pragma unroll
             for (int J = 0; J < NB; ++J) {
               ux[J] = fmaf(xv[J][e], dw[e], ux[J]);
@@ -249,12 +250,19 @@ __global__ __launch_bounds__(PT ? 64 * kLfPtWaves : (NB > 2 ? 256 : 64 * kLfMaxW
         }
         // the dot products stay here: moved to their use after the barrier they would hold every operand until then
 #pragma unroll
-        for (int I = 0; I < NB; ++I) asm volatile("" : "+v"(ux[I]), "+v"(vx[I]), "+v"(ug[I]));
+        for (int J = 0; J < NB; ++J) asm volatile("" : "+v"(ux[J]), "+v"(vx[J]), "+v"(ug[J]));
+        if (kHalf && k == 1) {
+          dm[0][0] += part[0][0];
+          part[0][0] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        }
       }
 #pragma unroll
-      for (int I = 0; I < IB; ++I)
-#pragma unroll
-        for (int J = 0; J < NB; ++J) dm[I0 + I][J] += part[I][J];
+      for (int J = 0; J < NB; ++J) {
+        if constexpr (kChains == 4) dm[I][J] += (part[0][J] + part[1][J]) + (part[2][J] + part[3][J]);
+        else if constexpr (kChains == 2) dm[I][J] += part[0][J] + part[1][J];
+        else dm[I][J] += part[0][J];
+      }
+      __builtin_amdgcn_sched_barrier(0);
     }
   };
   // M^T g of g[j] (n <= 32)

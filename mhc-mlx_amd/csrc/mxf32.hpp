@@ -321,35 +321,36 @@ void mxf_bwd_kernel(MxfArgs A) {
     for (int m = 0; m < NK; ++m) asm volatile("" : "+v"(yd[m]));  // formed here, not where the sums end
     issue_fence();
   };
-  // (the slab's products are summed by themselves first: one chain over all of a wave's slabs would round every product
-  // against the whole sum; see lf32_bwd.hpp)
+  // (a row block of G at a time, a slab's products in chains of 16: see lf32_bwd.hpp)
   auto sums = [&] {
-    f32x4 part[NB][NB];
 #pragma unroll
-    for (int I = 0; I < NB; ++I)
+    for (int I = 0; I < NB; ++I) {
+      f32x4 part[2][NB];
 #pragma unroll
-      for (int J = 0; J < NB; ++J) part[I][J] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+      for (int J = 0; J < NB; ++J) part[0][J] = part[1][J] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      __builtin_amdgcn_sched_barrier(0);
-      const int c = 16 * k + 4 * q;
-      f32x4 gv[NB], xv[NB];
+      for (int k = 0; k < 4; ++k) {
+        __builtin_amdgcn_sched_barrier(0);
+        const int c = 16 * k + 4 * q;
+        const f32x4 gv = *reinterpret_cast<const f32x4*>(sg + (16 * I + r) * kMxfPitch + c);
+        f32x4 xv[NB];
 #pragma unroll
-      for (int I = 0; I < NB; ++I) {
-        gv[I] = *reinterpret_cast<const f32x4*>(sg + (16 * I + r) * kMxfPitch + c);
-        xv[I] = *reinterpret_cast<const f32x4*>(sx + (16 * I + r) * kMxfPitch + c);
+        for (int J = 0; J < NB; ++J) xv[J] = *reinterpret_cast<const f32x4*>(sx + (16 * J + r) * kMxfPitch + c);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int J = 0; J < NB; ++J) part[e & 1][J] = lf_mfma(gv[e], xv[J][e], part[e & 1][J]);
+        if (k == 1) {
+#pragma unroll
+          for (int J = 0; J < NB; ++J) {
+            sm[I][J] += part[0][J] + part[1][J];
+            part[0][J] = part[1][J] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+          }
+        }
       }
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-#pragma unroll
-        for (int I = 0; I < NB; ++I)
-#pragma unroll
-          for (int J = 0; J < NB; ++J) part[I][J] = lf_mfma(gv[I][e], xv[J][e], part[I][J]);
+      for (int J = 0; J < NB; ++J) sm[I][J] += part[0][J] + part[1][J];
     }
-#pragma unroll
-    for (int I = 0; I < NB; ++I)
-#pragma unroll
-      for (int J = 0; J < NB; ++J) sm[I][J] += part[I][J];
   };
 
   int64_t s = (int64_t)blockIdx.x * kMxfWaves + wave;

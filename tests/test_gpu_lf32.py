@@ -129,3 +129,21 @@ def test_lf32_backward_activated_h(n, C):
     ref = torch.matmul(Md, xd) + pd[None, :, None] * yn[:, None, :]
     for g, r in zip(got, torch.autograd.grad(ref, ref_in, dev_tensor(dout).double())):
         assert rel_err(np_of(g), r.cpu().numpy()) < GRAD_TOL
+
+
+@pytest.mark.parametrize("T,n,C", [(130, 24, 100), (130, 32, 512), (600, 17, 512), (130, 48, 130), (130, 64, 512), (600, 40, 65)])
+def test_lf32_dM_is_as_exact_as_the_valu_kernels(T, n, C, knobs):
+    """dM at fp32 is no further from float64 than the VALU kernel's (MHC_BWD_MFMA=0): a slab's products are not one chain
+    of 64, which is 1.3 to 1.7 times as far.  The bound's 25% covers the spread of a norm over n^2 entries and the chains of
+    32 at n <= 32."""
+    g = rng(9200 + n)
+    x, dout = (dev_tensor(g.standard_normal((T, n, C))) for _ in range(2))
+    ps = [dev_tensor(v) for v in (g.uniform(size=(n, n)) / n, g.uniform(size=n), 2 * g.uniform(size=n), np.ones(C))]
+    ref = torch.matmul(dout.double().transpose(0, 1).reshape(n, -1), x.double().transpose(0, 1).reshape(n, -1).t())
+    err = []
+    for mfma in (1, 0):
+        knobs("MHC_BWD_MFMA", mfma)
+        M = ps[0].clone().requires_grad_(True)
+        out = ops.mhc_forward_fused_hip_autograd(x, M, *ps[1:], eps=EPS)
+        err.append(float((torch.autograd.grad(out, M, dout)[0] - ref).norm() / ref.norm()))
+    assert err[0] < 1.25 * err[1], err

@@ -103,3 +103,18 @@ def test_mxf32_rounds_no_more_than_its_sums_need(T, n, C):
         own = (M[:, k, None].astype(np.float64) * x[:, None, k] + own).astype(np.float32)
     own = own + y
     assert np.linalg.norm(out - ref) < 1.15 * np.linalg.norm(own - ref), np.linalg.norm(out - ref) / np.linalg.norm(own - ref)
+
+
+@pytest.mark.parametrize("T,n,C", [(300, 16, 100), (2000, 24, 20), (900, 32, 36), (600, 48, 100), (400, 64, 100)])
+def test_mxf32_dM_is_as_exact_as_the_valu_kernels(T, n, C, knobs):
+    """dM at fp32 is no further from float64 than the VALU kernel's (MHC_MIX32=0); see the layer's test of the same name."""
+    g = rng(9650 + n)
+    x, dout, y = (dev_tensor(g.standard_normal((T, n, C))) for _ in range(3))
+    ref = torch.matmul(dout.double().transpose(0, 1).reshape(n, -1), x.double().transpose(0, 1).reshape(n, -1).t())
+    err = []
+    for on in (1, 0):
+        knobs("MHC_MIX32", on)
+        M = dev_tensor(g.uniform(size=(n, n)) / n).requires_grad_(True)
+        out = ops.stream_mix_add_hip_autograd(x, M, y)
+        err.append(float((torch.autograd.grad(out, M, dout)[0] - ref).norm() / ref.norm()))
+    assert err[0] < 1.25 * err[1], err
