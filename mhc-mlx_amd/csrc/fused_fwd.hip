@@ -625,7 +625,7 @@ int launch_fwd_mfma16(FwdArgs A, hipStream_t stream) {
 }
 
 // Full-tile kernel for layer-wide n == NMAX <= 8.  Returns 1 when the shape
-// is not covered (the caller then uses fused_fwd_kernel).
+// is not covered.
 template <int NMAX, typename XT, typename OT>
 int launch_fwd_full(FwdArgs A, hipStream_t stream) {
   // A.vec (checked for 8-channel chunks) implies the alignment of narrower ones
@@ -670,6 +670,54 @@ int launch_fwd_full(FwdArgs A, hipStream_t stream) {
   return MHC_OK;
 }
 
+// Whether fused_fwd_kernel, one workgroup per token with its rows held in registers, takes a call at n <= 8 that the
+// narrow-token kernel (lv_fwd_kernel) would take too.  Measured, fused_fwd_kernel against lv_fwd_kernel:
+// * ragged rows (A.vec false): always the slower one;
+// * n > 4, C > 4096: lv reads x twice (625 x 8 x 8000 bf16 44 against 52 us);
+// * per token, n > 4, 16-bit output: lv's lanes run out of work against a token's 80 parameters (5000 x 8 x 1000 37
+//   against 41 us);
+// * per token, n > 4, fp32 output: at n = 5 lv's eight stream slots cost most (8000 x 5 x 3000 bf16 155 against 220 us,
+//   200 x 5 x 512 fp32 6.0 against 7.8); up to two tokens per CU, one wave per token leaves the CU idle (256 x 6 x 512
+//   fp32 6.4 against 7.7, 256 x 8 x 3072 20% the other way); rows that share 128-byte lines past 2048 channels (5714 x
+//   7 x 3000 157 against 202); narrow 16-bit rows (4096 x 6 x 64 31% apart, 32768 x 8 x 64 9% the other way); n = 6 with
+//   wide 16-bit rows (6510 x 6 x 3072 149 against 174, 6510 x 8 x 3072 equal);
+// * per token, n = 3 or 4, 16-bit output: beyond the caches (32768 x 4 x 4096 388 against 407, 16384 x 4 x 4096 192 against
+//   199, 8192 x 4 x 4096 equal), and 6144 channels in six waves (6510 x 3 x 6144 102 against 109);
+// * layer-wide, large calls: n = 5 and 6 where lv's chunks fill two, three or six waves or half its slots are padding
+//   (15625 x 5 x 1536 bf16 99 against 116, 8192 x 6 x 1536 to fp32 25% apart, 2000 x 5 x 1536 equal), and n = 3 at three or
+//   six waves (13020 x 3 x 3072 bf16 94 against 103, 2000 x 3 x 3072 10% the other way).
+template <typename XT, typename OT, bool PT>
+bool tile_fwd_first(const FwdArgs& A) {
+  if (!A.vec) return false;
+  constexpr bool half_x = sizeof(XT) == 2, half_out = sizeof(OT) == 2;
+  const int n = A.n, C = A.C;
+  if (n > 4 && C > 4096) return true;
+  const int64_t cus = device_cu_count(), T = A.T, chans = T * C;
+  const bool lines = (int64_t)C * sizeof(XT) % 128 == 0 && (int64_t)C * sizeof(OT) % 128 == 0;
+  if (PT && n > 4) {
+    if (half_out || n == 5) return true;
+    if (C > 2048 && !lines) return true;
+    if (T <= 2 * cus) return C >= 512 && (T <= cus / 2 || C < 1024 || (T <= cus && C < 2048));
+    if (C < 256) return T > 4 * cus && (n == 6 || (half_x && T <= 16 * cus));
+    return n == 6 && half_x && C > 1024 && T > 8 * cus;
+  }
+  if (PT) {
+    if (!half_out || n < 3) return false;
+    return lines && ((C > 2048 && C <= 4096 && chans * n > 150000000) || (C > 5120 && C <= 6144 && T > 8 * cus));
+  }
+  if (!half_x && n != 3) return false;
+  switch (n) {
+    case 3:
+      if (half_out && lines) return chans > 12000000 && ((C > 2048 && C <= 3072) || (C > 4096 && C <= 6144));
+      return !lines && C > 2048 && C <= 3072 && chans > 24000000;
+    case 5: return chans > 6000000 && C >= 768 && (half_out || (C > 1024 && C <= 2048));
+    case 6:
+      if (C > 1024 && C <= 1536) return chans > (half_out ? 12000000 : 6000000);
+      return half_out && C > 2048 && C <= 3072 && chans > 6000000;
+    default: return false;
+  }
+}
+
 template <int NMAX, typename XT, typename OT, bool PT>
 int launch_fwd(FwdArgs A, hipStream_t stream) {
   constexpr int V = FwdCfg<NMAX>::V;
@@ -679,13 +727,11 @@ int launch_fwd(FwdArgs A, hipStream_t stream) {
     const int rc = launch_fwd_full<NMAX, XT, OT>(A, stream);
     if (rc != 1) return rc;
   }
-  // What whole workgroups of whole chunks do not cover goes to the narrow-token kernel (forward, this kernel against
+  // What whole workgroups of whole chunks do not cover goes to the narrow-token kernel (forward, fused_fwd_kernel against
   // it: 9990 x 4 x 1001 bf16 103 against 36 us, 32768 x 4 x 96 bf16 37 against 14 us, per token 8192 x 4 x 4096 fp32 216
-  // against 186 us), except at n > 4 with whole vectors where that one would read x twice (625 x 8 x 8000 bf16 44
-  // against 52 us) or its lanes run out of work against a token's 80 parameters (per token, 16-bit output: 5000 x 8 x
-  // 1000 37 against 41 us).
+  // against 186 us), and to fused_fwd_kernel what that one declines or streams worse.
   if constexpr (NMAX <= 8) {
-    if (!(A.vec && A.n > 4 && (A.C > 4096 || (PT && ElemTraits<OT>::kBytes == 2)))) {
+    if (!tile_fwd_first<XT, OT, PT>(A)) {
       const int rc = lv_fused_fwd(gen_args(A), dtype_code<XT>(), dtype_code<OT>(), stream);
       if (rc != 1) return rc;
     }

@@ -10,9 +10,10 @@ import pytest
 import torch
 
 from oracle import mhc_oracle as O
-from tests._helpers import GRAD_TOL, TOL, dev_tensor, np_of, params, rel_err, rng, to_dtype_np
+from tests._helpers import GRAD_TOL, TOL, TORCH_DT, dev_tensor, np_of, params, rel_err, rng, to_dtype_np
 
 from mhc_mlx_amd import ops
+from mhc_mlx_amd.reference import mixing_matrix_from_logits
 
 pytestmark = pytest.mark.gpu
 
@@ -155,3 +156,40 @@ def test_lv_rounds_no_more_than_its_sums_need(T, n, C):
                 s = _fma(mat[i, k], rows[:, k], s)
             own[:, i] = _fma(scale[i], last, s)
         assert np.linalg.norm(got - ref) < 1.15 * np.linalg.norm(own - ref), np.linalg.norm(got - ref) / np.linalg.norm(own - ref)
+
+
+def _layer64(x, H, w):
+    """mhc_forward_reference in torch float64 on the GPU (large calls)."""
+    a, p, M = torch.sigmoid(H[0].double()), 2 * torch.sigmoid(H[1].double()), mixing_matrix_from_logits(H[2].double(), iters=20, eps=EPS)
+    y = (a.unsqueeze(-1) * x.double()).sum(-2)
+    yn = y * torch.rsqrt(y.square().mean(-1, keepdim=True) + EPS) * w.double()
+    return torch.matmul(M, x.double()) + p.unsqueeze(-1) * yn.unsqueeze(-2)
+
+
+# both sides of the lines at which the forward's dispatch changes kernels: tokens per CU, rows that share 128-byte lines,
+# channels, calls beyond the caches
+DISPATCH_FWD = [(200, 5, 512, "f32", "f32", True), (129, 6, 512, "bf16", "f32", True), (512, 8, 1000, "bf16", "f32", True),
+                (513, 8, 1000, "bf16", "f32", True), (300, 7, 3000, "f32", "f32", True), (300, 7, 3072, "f32", "f32", True),
+                (1100, 8, 64, "f16", "f32", True), (2100, 6, 1536, "bf16", "f32", True), (1300, 6, 136, "f32", "f32", True),
+                (2100, 3, 6144, "bf16", "bf16", True), (9200, 4, 4096, "bf16", "bf16", True),
+                (4100, 5, 1536, "bf16", "bf16", False), (4100, 5, 1536, "f16", "f32", False), (4000, 5, 1536, "bf16", "bf16", False),
+                (5000, 6, 1536, "bf16", "f32", False), (2100, 6, 3072, "bf16", "bf16", False), (4000, 3, 3072, "bf16", "bf16", False),
+                (8100, 3, 3000, "f32", "f32", False)]
+
+
+@pytest.mark.parametrize("T,n,C,xdt,odt,per_token", DISPATCH_FWD)
+def test_lv_forward_dispatch(T, n, C, xdt, odt, per_token):
+    g = torch.Generator(device="cuda")
+    g.manual_seed(T + n + C)
+    x = torch.randn(T, n, C, generator=g, device="cuda").to(TORCH_DT[xdt])
+    per = (T,) if per_token else ()
+    H = [torch.randn(*per, *s, generator=g, device="cuda") for s in ((n,), (n,), (n, n))]
+    w = 1 + 0.02 * torch.randn(C, generator=g, device="cuda")
+    fn = ops.mhc_layer_forward_dynamic if per_token else ops.mhc_layer_forward
+    with torch.no_grad():
+        out = fn(x, *H, w, sinkhorn_iters=20, eps=EPS, output_dtype=None if odt == "f32" else x.dtype)
+    assert out.dtype == TORCH_DT[odt]
+    for t in range(0, T, 1000):  # (in pieces: the reference is four times as wide)
+        part = slice(t, min(T, t + 1000))
+        ref = _layer64(x[part], [h[part] for h in H] if per_token else H, w)
+        assert float((out[part] - ref).abs().max() / ref.abs().max()) < TOL[odt]
