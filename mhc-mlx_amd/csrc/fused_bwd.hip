@@ -1498,9 +1498,8 @@ GenArgs gen_args(const BwdArgs& A, const BwdLayout& L) {
   return G;
 }
 
-// Layer-wide n <= 8 (fused_bwd_lw_kernel).  Returns 1 when the shape is not
-// covered (C too large for one chunk per thread), so the caller falls back
-// to fused_bwd_kernel.
+// n <= 8 (fused_bwd_lw_kernel).  Returns 1 when the shape is not covered (C
+// too large for one chunk per thread, or a partial tile that it does not take).
 template <int NMAX, typename XT, typename GT, bool PT>
 int launch_bwd_lw(BwdArgs A, const BwdLayout& L, int64_t* num_partials, hipStream_t stream) {
   constexpr int V = lw_vec<NMAX, XT, GT>();
@@ -1509,8 +1508,7 @@ int launch_bwd_lw(BwdArgs A, const BwdLayout& L, int64_t* num_partials, hipStrea
   if (tpb > lw_max_threads(NMAX)) return 1;
   const bool full = A.n == NMAX && A.vec && A.C % V == 0 && A.nchunks == tpb;
   // Partial tiles (n below NMAX, a partial last chunk or workgroup) run here only at n <= 4 with
-  // vector-aligned rows, on at most 512 threads (the variant's 256-VGPR bound); the others take the
-  // tile kernel, whose narrower chunks need less alignment.
+  // vector-aligned rows, on at most 512 threads (the variant's 256-VGPR bound).
   if (!full && (NMAX > 4 || !A.vec || tpb > 512)) return 1;
   // Grid: the workspace's full row budget (8 workgroups per CU) streams
   // faster than one resident wave of workgroups (562 vs 576 us at config 2);
@@ -1648,20 +1646,50 @@ int launch_bwd_tile(BwdArgs A, const BwdLayout& L, int64_t* num_partials, hipStr
 }
 
 // Whether fused_bwd_lw_kernel is asked before the narrow-token kernel of lv.hpp (each takes what the other declines).
-// Measured, backward kernel, lw against lv: layer-wide 16-bit rows of 2048 channels and more stream better on one
-// workgroup per token with its sums in registers (32768 x 4 x 4096 bf16 567 against 660 us, 8192 x 8 x 4096 365 against
-// 431 us; at C = 1024 163 against 147 us and 165 against 154 us, at C = 512 101 against 72 us); so do fp32 rows of 513 to
-// 1024 channels at n <= 4 (10000 x 4 x 1000 90 against 96 us; 8192 x 4 x 4096 280 against 276 us) and per-token 16-bit
-// rows of 1025 to 2048 channels at n = 8 (281 against 316 us).  Partial chunks per token, which lw would walk on the tile
-// kernel, all go to lv (4882 x 2 x 4096 fp32 210 against 89 us).
+// Measured, backward kernel, lw against lv:
+// * layer-wide, 16-bit rows of 2048 channels and more stream better on one workgroup per token with its sums in
+//   registers (32768 x 4 x 4096 bf16 567 against 660 us, 8192 x 8 x 4096 365 against 431 us; at C = 1024 163 against
+//   147 us and 165 against 154 us), at n = 4 from 1536 (19531 x 4 x 1536 128 against 135; 256 x 4 x 1536 18% the other
+//   way), at n = 8 also 512 and 1536 in large calls (29296 x 8 x 512 140 against 149, 9765 x 8 x 1536 166 against 175;
+//   4096 tokens 15% the other way);
+// * layer-wide, fp32 gradients, n <= 4: fp32 rows of 513 to 1024 channels (10000 x 4 x 1000 90 against 96 us; 8192 x 4 x
+//   4096 280 against 276 us) and, from 48 tokens per CU on, 512 channels and rows that share 128-byte lines up to 2048
+//   (30000 x 2 x 2000 261 against 289); 16-bit rows of 513 to 1024 there too (32768 x 4 x 768 138 against 151; 4096 x 4 x
+//   768 equal);
+// * per token, n = 8: 16-bit rows of 1025 to 2048 channels (281 against 316 us), and 512 or 1024 in large calls (14648 x
+//   8 x 1024 254 against 275; 2000 x 8 x 1024 equal);
+// * per token, n = 3 and 4: fp32 rows of 513 to 1024 channels at n = 4, and small calls, where its workgroups per token
+//   put more waves on a CU (200 x 4 x 1024 bf16 6.8 against 9.6 us, 256 x 4 x 8192 30%; 4096 x 4 x 4096 10% the other way).
+// Partial chunks per token, which lw would walk on the tile kernel, all go to lv (4882 x 2 x 4096 fp32 210 against 89 us).
 template <int NMAX, typename XT, typename GT, bool PT>
 bool lw_first(const BwdArgs& A) {
-  const bool pair16 = std::is_same<XT, GT>::value && sizeof(XT) == 2;
-  if (pair16) {
-    if (PT) return NMAX == 8 && A.n == NMAX && A.C > 1024 && A.C <= 2048;
-    return A.n == NMAX && A.C >= 2048;
+  constexpr bool pair16 = std::is_same<XT, GT>::value && sizeof(XT) == 2;
+  const int n = A.n, C = A.C;
+  const int64_t cus = device_cu_count(), T = A.T;
+  const bool full = n == NMAX && C % (pair16 ? 512 : 256) == 0;  // whole workgroups of whole chunks
+  if (PT && NMAX == 8) return pair16 && n == 8 && C <= 2048 && (C > 1024 || (full && T > 24 * cus));
+  if (PT && NMAX == 4) {
+    if (sizeof(XT) == 4 && n == 4 && C > 512 && C <= 1024) return true;
+    if (pair16) {
+      if (n == 3) return C == 1024 && T <= cus;
+      if (!full || C < 512) return false;
+      return C < 1024 ? T <= cus : (C <= 1536 ? T <= 16 * cus : T * C <= 1 << 21);
+    }
+    if (n < 3 || C % 256 != 0 || C < 512 || C > 2048) return false;
+    if (C > 512 && C <= 1024) return T <= 2 * cus;
+    return n == 4 && T <= (sizeof(XT) == 2 && C > 512 ? 2 : 1) * cus;
   }
-  return NMAX <= 4 && sizeof(XT) == 4 && A.C > 512 && A.C <= 1024 && (!PT || A.n == NMAX);
+  if (PT) return false;
+  if (pair16) {
+    if (n != NMAX) return false;
+    if (C >= 2048) return true;
+    if (NMAX == 4) return C == 1536 && T > 4 * cus;
+    return NMAX == 8 && full && C != 1024 && T > 32 * cus;
+  }
+  if (NMAX > 4) return false;
+  const bool many = T > 48 * cus;
+  if (C > 512 && C <= 1024) return sizeof(XT) == 4 || (many && n >= 3);
+  return many && sizeof(XT) == 4 && (C == 512 ? n == 4 : C > 1024 && C <= 2048 && C % 32 != 0);
 }
 
 template <int NMAX, typename XT, typename GT, bool PT>

@@ -193,3 +193,31 @@ def test_lv_forward_dispatch(T, n, C, xdt, odt, per_token):
         part = slice(t, min(T, t + 1000))
         ref = _layer64(x[part], [h[part] for h in H] if per_token else H, w)
         assert float((out[part] - ref).abs().max() / ref.abs().max()) < TOL[odt]
+
+
+DISPATCH_BWD = [(256, 4, 512, "bf16", "bf16", True), (257, 4, 512, "bf16", "bf16", True), (513, 4, 1024, "bf16", "bf16", True),
+                (300, 4, 6144, "bf16", "bf16", True), (345, 4, 6144, "f16", "f16", True), (200, 3, 1024, "bf16", "bf16", True),
+                (512, 3, 768, "bf16", "f32", True), (513, 3, 768, "f32", "f32", True), (400, 4, 2048, "f16", "f32", True),
+                (250, 4, 512, "f32", "f32", True), (6200, 8, 512, "bf16", "bf16", True),
+                (1100, 4, 1536, "bf16", "bf16", False), (1000, 4, 1536, "bf16", "bf16", False), (8200, 8, 512, "f16", "f16", False),
+                (12300, 4, 512, "f32", "f32", False), (12300, 2, 1100, "f32", "f32", False), (12300, 3, 520, "bf16", "f32", False)]
+
+
+@pytest.mark.parametrize("T,n,C,xdt,odt,per_token", DISPATCH_BWD)
+def test_lv_backward_dispatch(T, n, C, xdt, odt, per_token):
+    """Both sides of the lines at which the backward's dispatch changes kernels, every gradient against float64."""
+    g = torch.Generator(device="cuda")
+    g.manual_seed(T + n + C)
+    x = torch.randn(T, n, C, generator=g, device="cuda").to(TORCH_DT[xdt])
+    dout = torch.randn(T, n, C, generator=g, device="cuda").to(TORCH_DT[odt])
+    per = (T,) if per_token else ()
+    leaves = [x, *(torch.randn(*per, *s, generator=g, device="cuda") for s in ((n,), (n,), (n, n))),
+              1 + 0.02 * torch.randn(C, generator=g, device="cuda")]
+    fn = ops.mhc_layer_forward_dynamic if per_token else ops.mhc_layer_forward
+    ins = [t.clone().requires_grad_(True) for t in leaves]
+    out = fn(*ins, sinkhorn_iters=20, eps=EPS, output_dtype=None if odt == "f32" else x.dtype)
+    got = torch.autograd.grad(out, ins, dout)
+    ins = [t.double().requires_grad_(True) for t in leaves]
+    want = torch.autograd.grad(_layer64(ins[0], ins[1:4], ins[4]), ins, dout.double())
+    for name, a, r in zip(("dx", "dH_pre", "dH_post", "dH_res", "d_w"), got, want):
+        assert float((a - r).abs().max() / r.abs().max()) < (TOL[xdt] if name == "dx" else GRAD_TOL), name
