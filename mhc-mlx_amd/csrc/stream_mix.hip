@@ -832,9 +832,28 @@ int by_dtype(int code, F&& f) {
 
 // Whether the post-combine's MFMA kernels are asked first (they may decline).  They pad n to 16 rows: at n <= 4, and at
 // n <= 8 with whole aligned chunks, mix_add_*_kernel streams as fast or faster (8192 x 3 x 341 fp32 forward 33 against
-// 38 us); with ragged rows at n > 4 and everywhere above n = 8 the VALU kernel is the slower one (VJP call 8192 x 6 x 170
-// bf16 98 against 47 us, 8192 x 12 x 128 bf16 66 against 34 us).
-bool mxf_takes(int n, bool vec) { return n > 8 || (n > 4 && !vec); }
+// 38 us); with ragged rows at n > 4 the VALU kernel is the slower one (VJP call 8192 x 6 x 170 bf16 98 against 47 us).  At
+// 8 < n <= 16 it is too (8192 x 12 x 128 bf16 VJP 66 against 34 us), except in calls beyond the caches (`elems`, T n C:
+// below the lines the MFMA kernels are 2 to 60% ahead) whose rows share 128-byte lines (`lines` false): the forward to
+// fp32 (fp32 9090 x 12 x 1100 301 against 341 us, 2250 x 12 x 1100 equal; bf16 224 against 245, 2250 x 12 x 2000 14% the
+// other way) and the fp32 VJP (9090 x 12 x 1100 518 against 617 us, 1687 x 16 x 2000 10% the other way), at n = 16 that of
+// fp16 too (5681 x 16 x 1100 273 against 297); and in the 16-bit forward at n = 16 (2000 x 16 x 3000 125 against 143, 7324 x
+// 16 x 1024 126 against 134).
+bool mxf_takes(int n, bool vec, bool backward, int x_dtype, int o_dtype, bool lines, int64_t elems) {
+  if (n <= 8 || n > 16 || !vec) return n > 8 || (n > 4 && !vec);
+  const bool x_f32 = x_dtype == MHC_DTYPE_F32, o_f32 = o_dtype == MHC_DTYPE_F32;
+  if (backward) {
+    if (lines || !(x_f32 || (n == 16 && x_dtype == MHC_DTYPE_F16 && !o_f32))) return true;
+    return elems < (n == 16 ? 60000000 : 50000000);
+  }
+  if (!o_f32) return n < 16 || elems < 50000000;
+  return lines || elems < (x_f32 ? (n == 16 ? 33000000 : 50000000) : (n == 16 ? 47000000 : 80000000));
+}
+
+// rows of C channels that are whole 128-byte lines in every operand
+bool mix_lines(int C, int bx, int by, int bo) {
+  return (int64_t)C * bx % 128 == 0 && (int64_t)C * by % 128 == 0 && (int64_t)C * bo % 128 == 0;
+}
 
 int mix_rows(int n) { return round_up(n * n + n, 4); }
 
@@ -871,7 +890,8 @@ extern "C" int mhc_stream_mix_add_fwd(const void* x, int x_dtype, const void* y,
   Mix32Args F{};
   F.x = x; F.y = y; F.out = out; F.M = M; F.hpre = h_pre; F.hpost = h_post; F.T = T; F.n = n; F.C = C;
   F.h_mode = h_mode;
-  if (mxf_takes(n, A.vec)) {
+  if (mxf_takes(n, A.vec, false, x_dtype, out_dtype,
+                mix_lines(C, dtype_bytes(x_dtype), dtype_bytes(ydt), dtype_bytes(out_dtype)), T * n * C)) {
     int rc = mix32_fwd(F, x_dtype, ydt, out_dtype, s);
     if (rc != 1) return rc;
     rc = mxf_fwd(F, x_dtype, ydt, out_dtype, s);
@@ -948,7 +968,8 @@ extern "C" int mhc_stream_mix_add_bwd(const void* x, int x_dtype, const void* y,
   hipStream_t s = (hipStream_t)stream;
   int rc = 1;
   int64_t rows = G;  // partial rows written (the MFMA kernels choose their own count)
-  if (mxf_takes(n, A.vec)) {
+  if (mxf_takes(n, A.vec, true, x_dtype, dout_dtype,
+                mix_lines(C, dtype_bytes(x_dtype), dtype_bytes(ydt), dtype_bytes(dout_dtype)), T * n * C)) {
     Mix32Args F{};
     F.x = x; F.y = y; F.g = dout; F.out = dx; F.dy = dy; F.M = M; F.hpre = h_pre; F.hpost = h_post;
     F.part = (float*)workspace; F.T = T; F.n = n; F.C = C; F.h_mode = h_mode; F.P = P;

@@ -10,9 +10,10 @@ import pytest
 import torch
 
 from oracle import mhc_oracle as O
-from tests._helpers import GRAD_TOL, TOL, dev_tensor, np_of, params, rel_err, rng, to_dtype_np
+from tests._helpers import GRAD_TOL, TOL, TORCH_DT, dev_tensor, np_of, params, rel_err, rng, to_dtype_np
 
 from mhc_mlx_amd import ops
+from mhc_mlx_amd.reference import mixing_matrix_from_logits
 
 pytestmark = pytest.mark.gpu
 
@@ -118,3 +119,26 @@ def test_mxf32_dM_is_as_exact_as_the_valu_kernels(T, n, C, knobs):
         out = ops.stream_mix_add_hip_autograd(x, M, y)
         err.append(float((torch.autograd.grad(out, M, dout)[0] - ref).norm() / ref.norm()))
     assert err[0] < 1.25 * err[1], err
+
+
+@pytest.mark.parametrize("T,n,C,xdt,odt", [(4600, 12, 1000, "f32", "f32"), (2150, 16, 1000, "f32", "f32"), (2050, 16, 1000, "f32", "f32"),
+                                           (3800, 16, 1000, "f32", "f32"), (3800, 16, 1000, "bf16", "f32"),
+                                           (3100, 16, 1032, "bf16", "bf16"), (3800, 16, 1000, "f16", "f16"),
+                                           (3100, 16, 1024, "f32", "f32")])
+def test_mxf32_dispatch_of_large_calls(T, n, C, xdt, odt):
+    """8 < n <= 16 on both sides of the lines at which calls beyond the caches go to the VALU kernels, against float64."""
+    g = torch.Generator(device="cuda")
+    g.manual_seed(T + n)
+    R = lambda *s: torch.randn(*s, generator=g, device="cuda")  # noqa: E731
+    x, y, dout = R(T, n, C).to(TORCH_DT[xdt]), R(T, n, C).to(TORCH_DT[xdt]), R(T, n, C).to(TORCH_DT[odt])
+    hp, hq, hr = R(n), R(n), R(n, n)
+    ins = [t.clone().requires_grad_(True) for t in (x, y, hp, hq, hr)]
+    out = ops.post_combine(*ins, sinkhorn_iters=20, eps=1e-5, output_dtype=TORCH_DT[odt])
+    got = torch.autograd.grad(out, ins, dout)
+    ins = [t.double().requires_grad_(True) for t in (x, y, hp, hq, hr)]
+    M = mixing_matrix_from_logits(ins[4], iters=20, eps=1e-5) * torch.sigmoid(ins[2])
+    ref = 2 * torch.sigmoid(ins[3]).unsqueeze(-1) * (ins[1] + torch.matmul(M, ins[0]))
+    want = torch.autograd.grad(ref, ins, dout.double())
+    assert float((out.detach() - ref.detach()).abs().max() / ref.detach().abs().max()) < TOL[odt]
+    for name, a, r in zip(("dx", "dy", "dH_pre", "dH_post", "dH_res"), got, want):
+        assert float((a - r).abs().max() / r.abs().max()) < (TOL[xdt] if name in ("dx", "dy") else GRAD_TOL), name
