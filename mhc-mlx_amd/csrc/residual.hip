@@ -43,6 +43,7 @@ struct ResArgs {
   int h_mode;
   int vec;
   int P;
+  int tpb;
 };
 
 MHC_DEV float act_pre(const ResArgs& A, int i) {
@@ -106,14 +107,15 @@ __global__ __launch_bounds__(kResThreads) void residual_add_agg_kernel(ResArgs A
   const XT* X = (const XT*)A.x;
   const XT* R = (const XT*)A.res;
   OT* O = (OT*)A.out;
-  for (int64_t item0 = (int64_t)blockIdx.x * (kResThreads * K) + threadIdx.x; item0 < items;
-       item0 += (int64_t)gridDim.x * (kResThreads * K)) {
+  const int tpb = A.tpb;  // (an argument arrives with the others; blockDim costs a load of its own)
+  for (int64_t item0 = (int64_t)blockIdx.x * (tpb * K) + threadIdx.x; item0 < items;
+       item0 += (int64_t)gridDim.x * (tpb * K)) {
     int64_t base[K], to[K];
     bool in[K];
     float agg[K][V];
 #pragma unroll
     for (int k = 0; k < K; ++k) {
-      const int64_t item = item0 + k * kResThreads;
+      const int64_t item = item0 + k * tpb;
       in[k] = item < items;
       const int64_t t = items <= UINT32_MAX ? (int64_t)((uint32_t)item / (uint32_t)A.nchunks) : item / A.nchunks;
       const int c0 = (int)(item - t * A.nchunks) * V;
@@ -258,8 +260,8 @@ constexpr int kResBwdGroup = 4;
 // MI355X: 4% faster at 32768 x 4 x 4096 bf16 than the best of the persistent
 // grids of 2-32 blocks per CU.  MHC_RES_GRID > 0 caps the grid
 // at that many blocks per CU (tuning override).
-int64_t res_fwd_grid(int64_t items, int cus) {
-  const int64_t g = ceil_div(items, kResThreads);
+int64_t res_fwd_grid(int64_t items, int tpb, int cus) {
+  const int64_t g = ceil_div(items, tpb);
   const int per_cu = knob(kKnobResGrid, -1);
   if (per_cu < 0) return std::max<int64_t>(1, std::min<int64_t>(g, kMaxGrid));
   return std::max<int64_t>(1, std::min<int64_t>(g, (int64_t)cus * std::max(per_cu, 1)));
@@ -322,7 +324,15 @@ extern "C" int mhc_residual_add_agg_fwd(const void* x, const void* res, int dtyp
   // to fp32: 92 us cached, 95 with the hint).
   const bool nt = V > 1 && (int64_t)C * bx % 128 == 0 && (int64_t)C * bo % 128 == 0;
   A.nchunks = C / V;
-  const int64_t blocks = res_fwd_grid(ceil_div(T * A.nchunks, V > 1 ? 1 : res_group(n) > 4 ? 2 : 4), device_cu_count());
+  const int64_t lanes = ceil_div(T * A.nchunks, V > 1 ? 1 : res_group(n) > 4 ? 2 : 4);
+  // One wave per workgroup where four leave half the CUs without work or a few with twice the work of the rest (200 x 9 x
+  // 1536 fp32, 300 workgroups of four waves 8.3 us, 1200 of one 6.6; 400 x 48 x 768 39.6 and 31); elsewhere four (400 x 4 x
+  // 1536, 600 workgroups, equal; 2000 x 2 x 768 bf16 5.0 against 6.3), and at n < 4, where a wave has few loads to wait for.
+  const int cus = device_cu_count();
+  const int64_t wide = ceil_div(lanes, kResThreads);
+  const int tpb = n >= 4 && (2 * wide <= cus || (wide > cus && 4 * wide <= 5 * (int64_t)cus)) ? 64 : kResThreads;
+  A.tpb = tpb;
+  const int64_t blocks = res_fwd_grid(lanes, tpb, cus);
   hipStream_t s = (hipStream_t)stream;
   return res_by_group(n, [&](auto gc) {
     constexpr int G = decltype(gc)::value;
@@ -332,7 +342,7 @@ extern "C" int mhc_residual_add_agg_fwd(const void* x, const void* res, int dtyp
         using OT = std::remove_pointer_t<decltype(op)>;
         auto go = [&](auto vc, auto ntc) {
           hipLaunchKernelGGL((residual_add_agg_kernel<G, XT, OT, decltype(vc)::value, decltype(ntc)::value>),
-                             dim3((unsigned)blocks), dim3(kResThreads), 0, s, A);
+                             dim3((unsigned)blocks), dim3(tpb), 0, s, A);
           MHC_CHECK_LAUNCH("residual_add_agg_kernel");
           return (int)MHC_OK;
         };

@@ -66,6 +66,18 @@ def test_forward_widths(B, n, C, xdt, odt, shift, grid, knobs):
     assert rel_err(np_of(y), O.residual_add_agg(x, res, h)[1]) < 1e-5
 
 
+@pytest.mark.parametrize("B,n,C", [(300, 3, 512), (200, 9, 1536), (700, 2, 1024), (450, 3, 1001)])
+@pytest.mark.parametrize("grid", [None, 1])
+def test_forward_workgroups_of_one_and_four_waves(B, n, C, grid, knobs):
+    """Fewer workgroups of four waves than CUs, a few more, and many more (one wave each in the second)."""
+    if grid is not None:
+        knobs("MHC_RES_GRID", grid)
+    x, res, h = _inputs(B, n, C, "f32", 19 + B)
+    out, y = ops.residual_add_agg_hip(dev_tensor(x), dev_tensor(res), dev_tensor(h))
+    ro, ry = O.residual_add_agg(x, res, h)
+    assert rel_err(np_of(out), ro) < 1e-6 and rel_err(np_of(y), ry) < 1e-5
+
+
 @pytest.mark.parametrize("xdt", ["f32", "bf16", "f16"])
 @pytest.mark.parametrize("odt", ["bf16", "f16"])
 def test_half_output_is_rounded_sum(xdt, odt):
