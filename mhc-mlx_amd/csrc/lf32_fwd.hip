@@ -372,10 +372,15 @@ int lf32_fused_fwd(const GenArgs& A, int xd, int od, hipStream_t s) {
   if (knob(kKnobFwdMfma, 1) == 0) return 1;
   // offsets inside a token are 32-bit, with the top bit for "outside"
   if ((int64_t)A.n * A.C * 4 >= (int64_t)1 << 31 || A.n > 64) return 1;
-  // fp32 rows of 25 to 32 slabs at n <= 16: four slabs per wave leave one workgroup per CU, and fused_fwd_kernel, one
-  // pass on up to 1024 threads, is the faster one (1000 x 12 x 2000 39.6 against 46.5 us; at C = 1500 47.8 against
-  // 45.9 us, at C = 3000, where it reads x twice, 81.9 against 63.6 us)
-  if (A.n <= 16 && xd == MHC_DTYPE_F32 && A.C > 1536 && A.C <= 2048) return 1;
+  // fp32 rows of 21 to 32 slabs at n <= 16, one element at a time (ragged or unaligned), are read twice here, and
+  // fused_fwd_kernel, one pass on up to 1024 threads, is the faster one once the CUs have tokens enough (4000 x 12 x 1999
+  // 190 against 228 us, 300 x 12 x 1999 22 against 18; 3000 x 16 x 1301 137 against 150, 1000 x 9 x 1301 27 against 22).
+  // Vector rows, four slabs per wave, are not (4000 x 12 x 2000 157 against 150, 3000 x 16 x 2048 149 against 132, per token
+  // 3000 x 9 x 1600 83 against 68).
+  if (A.n <= 16 && xd == MHC_DTYPE_F32 && A.C > 1280 && A.C <= 2048 &&
+      A.T > (A.C > 1536 ? 2 : 8) * (int64_t)device_cu_count() &&
+      lf_mode(A.C, 4, 4, aligned(A.x, 16) && aligned(A.out, 16)) == kLfElem)
+    return 1;
   if (xd == MHC_DTYPE_F32 && od == MHC_DTYPE_F32) return lf_fwd_types<float, float>(A, s);
   if (xd == MHC_DTYPE_BF16 && od == MHC_DTYPE_F32) return lf_fwd_types<__bf16, float>(A, s);
   if (xd == MHC_DTYPE_BF16 && od == MHC_DTYPE_BF16) return lf_fwd_types<__bf16, __bf16>(A, s);

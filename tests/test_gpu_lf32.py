@@ -18,7 +18,7 @@ from mhc_mlx_amd import ops
 pytestmark = pytest.mark.gpu
 
 EPS = 1e-5
-SHAPES = [(3, 9, 4), (70, 16, 64), (5, 16, 68), (300, 12, 100), (7, 16, 516), (4, 13, 1100), (3, 16, 2304),
+SHAPES = [(3, 9, 4), (4, 12, 1999), (3, 16, 2000), (70, 16, 64), (5, 16, 68), (300, 12, 100), (7, 16, 516), (4, 13, 1100), (3, 16, 2304),
           (40, 17, 65), (9, 32, 512), (6, 32, 516), (3, 24, 1030), (5, 32, 1096), (2, 20, 2500),
           (4, 33, 61), (6, 48, 512), (3, 49, 130), (5, 64, 192), (2, 64, 1000), (2, 40, 516)]
 
