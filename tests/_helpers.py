@@ -5,6 +5,8 @@ import torch
 
 from oracle import mhc_oracle as O
 
+from mhc_mlx_amd.reference import mixing_matrix_from_logits
+
 TORCH_DT = {"f32": torch.float32, "bf16": torch.bfloat16, "f16": torch.float16}
 
 
@@ -66,3 +68,21 @@ def params(g: np.random.Generator, n: int, C: int, per_token_B: int | None = Non
     hres = g.standard_normal(shp + (n,)).astype(np.float32)
     w = (1.0 + 0.02 * g.standard_normal(C)).astype(np.float32)
     return hpre, hpost, hres, w
+
+
+def layer64(x, H, w, eps=1e-5, iters=20):
+    """mhc_forward_reference (reference.py:164-184) in torch float64 on x's device, for calls too large for numpy."""
+    a, p = torch.sigmoid(H[0].double()), 2 * torch.sigmoid(H[1].double())
+    M = mixing_matrix_from_logits(H[2].double(), iters=iters, eps=eps)
+    y = (a.unsqueeze(-1) * x.double()).sum(-2)
+    yn = y * torch.rsqrt(y.square().mean(-1, keepdim=True) + eps) * w.double()
+    return torch.matmul(M, x.double()) + p.unsqueeze(-1) * yn.unsqueeze(-2)
+
+
+def kernels_missing(fn, *names: str) -> list[str]:
+    """Those of `names` that are no part of the name of any kernel that fn() launches."""
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+        fn()
+        torch.cuda.synchronize()
+    ran = [e.key for e in prof.key_averages()]
+    return [n for n in names if not any(n in k for k in ran)]

@@ -10,17 +10,16 @@ import pytest
 import torch
 
 from oracle import mhc_oracle as O
-from tests._helpers import GRAD_TOL, TOL, TORCH_DT, dev_tensor, np_of, params, rel_err, rng, to_dtype_np
+from tests._helpers import GRAD_TOL, TOL, TORCH_DT, dev_tensor, kernels_missing, layer64, np_of, params, rel_err, rng, to_dtype_np
 
 from mhc_mlx_amd import ops
-from mhc_mlx_amd.reference import mixing_matrix_from_logits
 
 pytestmark = pytest.mark.gpu
 
 EPS = 1e-5
 SHAPES = [(37, 2, 1), (19, 3, 16), (70, 4, 64), (33, 4, 65), (18, 8, 100), (9, 5, 128), (21, 1, 132), (5, 2, 300),
           (7, 4, 777), (3, 6, 1000), (6, 4, 1040), (4, 8, 1030), (3, 2, 2056), (2, 3, 4100), (2, 8, 2500), (3, 4, 8008),
-          (2, 4, 9001), (2, 7, 4200)]
+          (2, 4, 9001), (2, 7, 4200), (3, 7, 2501)]
 
 
 @pytest.mark.parametrize("T,n,C", SHAPES)
@@ -28,7 +27,7 @@ SHAPES = [(37, 2, 1), (19, 3, 16), (70, 4, 64), (33, 4, 65), (18, 8, 100), (9, 5
 @pytest.mark.parametrize("per_token", [False, True])
 @pytest.mark.parametrize("grid", [None, 1])
 def test_lv_forward_and_backward(T, n, C, xdt, odt, per_token, grid, knobs):
-    """Output and every gradient, on the whole chip and on one workgroup (per CU) that walks every token; reruns are
+    """Output and every gradient, the backward on the whole chip and on one workgroup that walks every token; reruns are
     bitwise equal."""
     if grid is not None:
         knobs("MHC_FWD_GRID", grid)
@@ -83,7 +82,6 @@ def test_lv_matches_the_tile_kernel(n, C, knobs):
     for other in res[1:]:
         for a, b in zip(res[0], other):
             assert rel_err(np_of(a), np_of(b)) < 1e-5
-    assert not all(torch.equal(a, b) for a, b in zip(res[0][1:], res[2][1:]))
 
 
 @pytest.mark.parametrize("T,n,C", [(37, 4, 64), (1, 2, 33), (18, 8, 100), (5, 3, 128), (37, 4, 200), (3, 4, 777)])
@@ -158,14 +156,6 @@ def test_lv_rounds_no_more_than_its_sums_need(T, n, C):
         assert np.linalg.norm(got - ref) < 1.15 * np.linalg.norm(own - ref), np.linalg.norm(got - ref) / np.linalg.norm(own - ref)
 
 
-def _layer64(x, H, w):
-    """mhc_forward_reference in torch float64 on the GPU (large calls)."""
-    a, p, M = torch.sigmoid(H[0].double()), 2 * torch.sigmoid(H[1].double()), mixing_matrix_from_logits(H[2].double(), iters=20, eps=EPS)
-    y = (a.unsqueeze(-1) * x.double()).sum(-2)
-    yn = y * torch.rsqrt(y.square().mean(-1, keepdim=True) + EPS) * w.double()
-    return torch.matmul(M, x.double()) + p.unsqueeze(-1) * yn.unsqueeze(-2)
-
-
 # both sides of the lines at which the forward's dispatch changes kernels: tokens per CU, rows that share 128-byte lines,
 # channels, calls beyond the caches
 DISPATCH_FWD = [(200, 5, 512, "f32", "f32", True), (129, 6, 512, "bf16", "f32", True), (512, 8, 1000, "bf16", "f32", True),
@@ -191,7 +181,7 @@ def test_lv_forward_dispatch(T, n, C, xdt, odt, per_token):
     assert out.dtype == TORCH_DT[odt]
     for t in range(0, T, 1000):  # (in pieces: the reference is four times as wide)
         part = slice(t, min(T, t + 1000))
-        ref = _layer64(x[part], [h[part] for h in H] if per_token else H, w)
+        ref = layer64(x[part], [h[part] for h in H] if per_token else H, w)
         assert float((out[part] - ref).abs().max() / ref.abs().max()) < TOL[odt]
 
 
@@ -218,6 +208,54 @@ def test_lv_backward_dispatch(T, n, C, xdt, odt, per_token):
     out = fn(*ins, sinkhorn_iters=20, eps=EPS, output_dtype=None if odt == "f32" else x.dtype)
     got = torch.autograd.grad(out, ins, dout)
     ins = [t.double().requires_grad_(True) for t in leaves]
-    want = torch.autograd.grad(_layer64(ins[0], ins[1:4], ins[4]), ins, dout.double())
+    want = torch.autograd.grad(layer64(ins[0], ins[1:4], ins[4]), ins, dout.double())
     for name, a, r in zip(("dx", "dH_pre", "dH_post", "dH_res", "d_w"), got, want):
         assert float((a - r).abs().max() / r.abs().max()) < (TOL[xdt] if name == "dx" else GRAD_TOL), name
+
+
+@pytest.mark.parametrize("T,n,C,xdt", [(9000, 3, 33, "f32"), (9000, 4, 64, "bf16"), (4500, 4, 100, "f32"), (2300, 4, 260, "bf16"),
+                                       (2300, 8, 200, "f32"), (700, 2, 777, "f16"), (700, 4, 1040, "f32"), (560, 7, 1030, "f32"),
+                                       (530, 3, 4100, "bf16"), (530, 8, 2501, "f32")])
+@pytest.mark.parametrize("per_token", [False, True])
+def test_lv_forward_walks_its_tokens(T, n, C, xdt, per_token, knobs):
+    """One workgroup per CU: every wave (16, 32 or 64 lanes per token) or workgroup (two and more waves per token) takes
+    two tokens at least, so the reduction buffers alternate and per-token parameters are loaded again."""
+    knobs("MHC_FWD_GRID", 1)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    vec = 8 if xdt != "f32" and C % 8 == 0 else 4
+    lanes = 64 if per_token or C > 32 * vec else (32 if C > 16 * vec else 16)
+    assert T > 2 * cus * (4 * (64 // lanes) if C <= 64 * vec else 1)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(T + n + C)
+    x = torch.randn(T, n, C, generator=g, device="cuda").to(TORCH_DT[xdt])
+    per = (T,) if per_token else ()
+    H = [torch.randn(*per, *s, generator=g, device="cuda") for s in ((n,), (n,), (n, n))]
+    w = 1 + 0.02 * torch.randn(C, generator=g, device="cuda")
+    fn = ops.mhc_layer_forward_dynamic if per_token else ops.mhc_layer_forward
+    with torch.no_grad():
+        out = fn(x, *H, w, sinkhorn_iters=20, eps=EPS)
+    ref = layer64(x, H, w, EPS)
+    assert float((out - ref).abs().max() / ref.abs().max()) < 1e-5
+
+
+@pytest.mark.parametrize("T,n,C,xdt,per_token,fwd,bwd", [
+    (37, 4, 64, "f32", False, "lv_fwd_kernel", "lv_bwd_kernel"),
+    (9, 4, 1001, "bf16", True, "lv_fwd_kernel", "lv_bwd_kernel"),
+    (9, 8, 2501, "f32", False, "lv_fwd_kernel", "lv_bwd_kernel"),
+    (9, 7, 2501, "bf16", False, "lv_fwd_kernel", "bwd_tile_kernel"),  # two 16-bit operands element by element, n > 4, C > 2048
+    (9, 5, 1000, "f32", True, "fused_fwd_kernel", "lv_bwd_kernel"),
+    (9, 4, 1024, "bf16", True, "lv_fwd_kernel", "fused_bwd_lw_kernel"),
+    (9, 4, 4096, "bf16", False, "fused_fwd_full_kernel", "fused_bwd_lw_kernel")])
+def test_lv_kernels_run(T, n, C, xdt, per_token, fwd, bwd):
+    """Which kernels take a call, in each direction (outputs of x's dtype)."""
+    per = (T,) if per_token else ()
+    x = torch.randn(T, n, C, device="cuda").to(TORCH_DT[xdt]).requires_grad_(True)
+    H = [torch.randn(*per, *s, device="cuda").requires_grad_(True) for s in ((n,), (n,), (n, n))]
+    w = torch.ones(C, device="cuda").requires_grad_(True)
+    fn = ops.mhc_layer_forward_dynamic if per_token else ops.mhc_layer_forward
+
+    def step():
+        out = fn(x, *H, w, eps=EPS, output_dtype=x.dtype)
+        torch.autograd.grad(out, [x, *H, w], torch.ones_like(out))
+
+    assert not kernels_missing(step, fwd, bwd)

@@ -10,7 +10,7 @@ import pytest
 import torch
 
 from oracle import mhc_oracle as O
-from tests._helpers import GRAD_TOL, TOL, TORCH_DT, dev_tensor, np_of, params, rel_err, rng, to_dtype_np
+from tests._helpers import GRAD_TOL, TOL, TORCH_DT, dev_tensor, kernels_missing, np_of, params, rel_err, rng, to_dtype_np
 
 from mhc_mlx_amd import ops
 from mhc_mlx_amd.reference import mixing_matrix_from_logits
@@ -50,12 +50,16 @@ def test_mxf32_post_combine(T, n, C, xdt, odt, grid, knobs):
         assert rel_err(np_of(a), r, floor=1e-3) < tol, (name, rel_err(np_of(a), r))
 
 
-@pytest.mark.parametrize("T,n,C", [(900, 24, 20), (4000, 12, 7), (700, 40, 12)])
+@pytest.mark.parametrize("T,n,C", [(8000, 12, 20), (21000, 12, 7), (4500, 12, 32), (8000, 24, 20), (4500, 24, 32), (21000, 24, 7),
+                                   (8000, 40, 20), (4500, 64, 32)])
 def test_mxf32_many_slabs_per_wave(T, n, C, knobs):
-    """Two workgroups' worth of rows: every wave walks many slabs and the sums match the VALU kernels' (MHC_MIX32=0)."""
-    g = rng(9400 + T)
-    x, y, dout = (dev_tensor(g.standard_normal((T, n, C))) for _ in range(3))
-    M = dev_tensor(g.uniform(size=(n, n)))
+    """One workgroup per CU: every wave walks two slabs at least, the next one's loads ahead of this one's rows; against
+    float64 and the VALU kernels (MHC_MIX32=0)."""
+    assert T * C // 64 > 2 * 4 * torch.cuda.get_device_properties(0).multi_processor_count
+    g = torch.Generator(device="cuda")
+    g.manual_seed(T + n)
+    x, y, dout = (torch.randn(T, n, C, generator=g, device="cuda") for _ in range(3))
+    M = torch.rand(n, n, generator=g, device="cuda")
     res = []
     for on in (1, 0):
         knobs("MHC_MIX32", on)
@@ -64,9 +68,32 @@ def test_mxf32_many_slabs_per_wave(T, n, C, knobs):
         ts = [t.clone().requires_grad_(True) for t in (x, M, y)]
         out = ops.stream_mix_add_hip_autograd(*ts)
         res.append([out.detach(), *torch.autograd.grad(out, ts, dout)])
-    for a, b in zip(*res):
-        assert rel_err(np_of(a), np_of(b)) < 1e-5
-    assert not torch.equal(res[0][2], res[1][2])
+    ts = [t.double().requires_grad_(True) for t in (x, M, y)]
+    out = torch.matmul(ts[1], ts[0]) + ts[2]
+    res.append([out.detach(), *torch.autograd.grad(out, ts, dout.double())])
+    for a, b, r in zip(*res):
+        assert float((a - r).abs().max() / r.abs().max()) < 1e-5
+        assert float((a - b).abs().max() / r.abs().max()) < 1e-5
+
+
+@pytest.mark.parametrize("n,C", [(6, 31), (12, 4), (20, 20), (40, 12), (64, 1)])
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_mxf32_keeps_non_finite_values_in_their_channel(n, C, bad):
+    """A slab holds several tokens: an infinity or a NaN of x reaches its own token and channel of out, one of dout those
+    of dx and dy."""
+    T, t, c = 33, 16, C // 2
+    g = rng(9700 + n)
+    x, y, dout = (dev_tensor(g.standard_normal((T, n, C))) for _ in range(3))
+    x[t, 1, c] = dout[t, n - 1, c] = bad
+    M = dev_tensor(g.uniform(size=(n, n)))
+    ts = [v.requires_grad_(True) for v in (x, M, y)]
+    out = ops.stream_mix_add_hip_autograd(*ts)
+    dx, _, dy = torch.autograd.grad(out, ts, dout)
+    for v in (out, dx, dy):
+        broken = ~torch.isfinite(v)
+        assert broken[t, :, c].any()
+        broken[t, :, c] = False
+        assert not broken.any()
 
 
 def test_mxf32_unaligned_rows():
@@ -142,3 +169,15 @@ def test_mxf32_dispatch_of_large_calls(T, n, C, xdt, odt):
     assert float((out.detach() - ref.detach()).abs().max() / ref.detach().abs().max()) < TOL[odt]
     for name, a, r in zip(("dx", "dy", "dH_pre", "dH_post", "dH_res"), got, want):
         assert float((a - r).abs().max() / r.abs().max()) < (TOL[xdt] if name in ("dx", "dy") else GRAD_TOL), name
+
+
+@pytest.mark.parametrize("T,n,C", [(3, 5, 3), (9, 16, 64), (11, 17, 32), (2, 48, 76), (3, 64, 20)])
+def test_mxf32_kernels_run(T, n, C):
+    """The shapes above are the fp32-MFMA kernels' in both directions."""
+    ts = [torch.randn(*s, device="cuda").requires_grad_(True) for s in ((T, n, C), (n, n), (T, n, C))]
+
+    def step():
+        out = ops.stream_mix_add_hip_autograd(*ts)
+        torch.autograd.grad(out, ts, torch.ones_like(out))
+
+    assert not kernels_missing(step, "mxf_fwd_kernel", "mxf_bwd_kernel")
