@@ -1,6 +1,9 @@
 // The layer at n <= 8 on the VALU for rows of any width and alignment: what
 // fused_fwd_full_kernel and fused_bwd_lw_kernel (whole aligned chunks, whole
-// workgroups) do not take.  At n <= 8 the mix is at most 64 FMAs per channel
+// workgroups) do not take, less what tile_fwd_first (fused_fwd.hip) keeps on
+// fused_fwd_kernel, and in the backward two 16-bit operands element by element
+// over more than 2048 channels of more than four streams (one offset per
+// element of both does not fit the registers: bwd_tile_kernel).  At n <= 8 the mix is at most 64 FMAs per channel
 // and HBM is the bound as long as every byte moves once, in wide accesses,
 // with every lane at work, so:
 //
@@ -26,7 +29,8 @@
 // 9990 x 4 x 1001 bf16 164 -> 53 us, 4882 x 2 x 4096 bf16 108 -> 51 us, 32768 x
 // 8 x 96 bf16 529 -> 41 us, 833 x 6 x 8000 bf16 213 -> 99 us (its 96 sums hold
 // two waves per SIMD), per token 32768 x 8 x 96 bf16 637 -> 141 us and 8192 x 4 x
-// 4096 bf16 179 -> 159 us (5.1 TB/s).
+// 4096 bf16 179 -> 161 us (5.1 TB/s) repeated on the same tensors (185 us in a
+// training step's trace, behind the forward and the Sinkhorn VJP).
 #pragma once
 
 #include <type_traits>
@@ -773,16 +777,21 @@ int lv_fwd_typed(const GenArgs& A, hipStream_t s) {
         constexpr int SPW = decltype(sp)::value, G = decltype(gr)::value;
         auto go = [&](auto ptc) {
           constexpr bool PT = decltype(ptc)::value;
-          const int tpb = lv_threads(wpt);
-          const int occ = occupancy_blocks((const void*)lv_fwd_kernel<NM, XT, OT, MODE, SPW, G, PT>, tpb, 0);
-          if (occ <= 0) return 1;
-          const int per_cu = knob(kKnobFwdGrid, 0);
-          int64_t blocks = (int64_t)device_cu_count() * (per_cu > 0 ? per_cu : occ);
-          blocks = std::max<int64_t>(1, std::min(blocks, ceil_div(A.T, lv_tokens(wpt, G))));
-          hipLaunchKernelGGL((lv_fwd_kernel<NM, XT, OT, MODE, SPW, G, PT>), dim3((unsigned)blocks), dim3(tpb), 0, s,
-                             GenFwdArgs(A), wpt);
-          MHC_CHECK_LAUNCH("lv_fwd_kernel");
-          return (int)MHC_OK;
+          // (at n > 4 whole vectors of 16-bit rows go to fused_fwd_kernel per token and past 4096 channels)
+          if constexpr (NM > 4 && (MODE & 3) == kLvOct && (PT || SPW == 0)) {
+            return 1;
+          } else {
+            const int tpb = lv_threads(wpt);
+            const int occ = occupancy_blocks((const void*)lv_fwd_kernel<NM, XT, OT, MODE, SPW, G, PT>, tpb, 0);
+            if (occ <= 0) return 1;
+            const int per_cu = knob(kKnobFwdGrid, 0);
+            int64_t blocks = (int64_t)device_cu_count() * (per_cu > 0 ? per_cu : occ);
+            blocks = std::max<int64_t>(1, std::min(blocks, ceil_div(A.T, lv_tokens(wpt, G))));
+            hipLaunchKernelGGL((lv_fwd_kernel<NM, XT, OT, MODE, SPW, G, PT>), dim3((unsigned)blocks), dim3(tpb), 0, s,
+                               GenFwdArgs(A), wpt);
+            MHC_CHECK_LAUNCH("lv_fwd_kernel");
+            return (int)MHC_OK;
+          }
         };
         if constexpr (G == 64) {
           if (pt) return go(std::true_type{});

@@ -79,6 +79,35 @@ def layer64(x, H, w, eps=1e-5, iters=20):
     return torch.matmul(M, x.double()) + p.unsqueeze(-1) * yn.unsqueeze(-2)
 
 
+def tokens_dot(a, b):
+    """sum over tokens and channels of a[t, i, c] b[t, j, c], as one matrix product.  (torch's sum over many blocks in
+    float64 has given a wrong value on the GPU now and then, so references form their long sums this way.)"""
+    def rows(t):
+        return t.transpose(0, 1).reshape(t.shape[1], -1)
+
+    return torch.matmul(rows(a), rows(b).t().contiguous())
+
+
+def layer_grads64(x, H, w, dout, eps=1e-5, iters=20):
+    """(dx, dH_pre, dH_post, dH_res, d_w) of layer64 for the cotangent dout, in torch float64 on x's device."""
+    per_token, C = H[0].dim() == 2, x.shape[2]
+    H = [h.detach().double().requires_grad_(True) for h in H]
+    act = torch.sigmoid(H[0]), 2 * torch.sigmoid(H[1]), mixing_matrix_from_logits(H[2], iters=iters, eps=eps)
+    a, p, M = (t.detach() for t in act)
+    x, g, w = x.detach().double(), dout.double(), w.detach().double()
+    y, d = (a.unsqueeze(-1) * x).sum(-2), (p.unsqueeze(-1) * g).sum(-2)
+    inv = torch.rsqrt(y.square().mean(-1, keepdim=True) + eps)
+    dy = d * inv * w - inv ** 3 / C * (d * y * w).sum(-1, keepdim=True) * y
+    yn = y * inv * w
+    dx = torch.matmul(M.transpose(-1, -2).contiguous(), g) + a.unsqueeze(-1) * dy.unsqueeze(-2)
+    dw = torch.matmul(torch.ones(1, x.shape[0], dtype=x.dtype, device=x.device), d * y * inv)[0]
+    if per_token:
+        sums = ((dy.unsqueeze(-2) * x).sum(-1), (g * yn.unsqueeze(-2)).sum(-1), torch.matmul(g, x.transpose(-1, -2).contiguous()))
+    else:
+        sums = tokens_dot(x, dy.unsqueeze(1))[:, 0], tokens_dot(g, yn.unsqueeze(1))[:, 0], tokens_dot(g, x)
+    return (dx, *torch.autograd.grad(act, H, sums), dw)
+
+
 def kernels_missing(fn, *names: str) -> list[str]:
     """Those of `names` that are no part of the name of any kernel that fn() launches."""
     with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:

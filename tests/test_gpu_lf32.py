@@ -11,7 +11,8 @@ import pytest
 import torch
 
 from oracle import mhc_oracle as O
-from tests._helpers import GRAD_TOL, TOL, TORCH_DT, dev_tensor, kernels_missing, layer64, np_of, params, rel_err, rng, to_dtype_np
+from tests._helpers import (GRAD_TOL, TOL, TORCH_DT, dev_tensor, kernels_missing, layer64, np_of, params,
+                            rel_err, rng, to_dtype_np, tokens_dot)
 
 from mhc_mlx_amd import ops
 
@@ -132,7 +133,7 @@ def test_lf32_dM_is_as_exact_as_the_valu_kernels(T, n, C, knobs):
     g = rng(9200 + n)
     x, dout = (dev_tensor(g.standard_normal((T, n, C))) for _ in range(2))
     ps = [dev_tensor(v) for v in (g.uniform(size=(n, n)) / n, g.uniform(size=n), 2 * g.uniform(size=n), np.ones(C))]
-    ref = torch.matmul(dout.double().transpose(0, 1).reshape(n, -1), x.double().transpose(0, 1).reshape(n, -1).t())
+    ref = tokens_dot(dout.double(), x.double())
     err = []
     for mfma in (1, 0):
         knobs("MHC_BWD_MFMA", mfma)

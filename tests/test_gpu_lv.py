@@ -10,7 +10,8 @@ import pytest
 import torch
 
 from oracle import mhc_oracle as O
-from tests._helpers import GRAD_TOL, TOL, TORCH_DT, dev_tensor, kernels_missing, layer64, np_of, params, rel_err, rng, to_dtype_np
+from tests._helpers import (GRAD_TOL, TOL, TORCH_DT, dev_tensor, kernels_missing, layer64, layer_grads64,
+                            np_of, params, rel_err, rng, to_dtype_np)
 
 from mhc_mlx_amd import ops
 
@@ -207,8 +208,7 @@ def test_lv_backward_dispatch(T, n, C, xdt, odt, per_token):
     ins = [t.clone().requires_grad_(True) for t in leaves]
     out = fn(*ins, sinkhorn_iters=20, eps=EPS, output_dtype=None if odt == "f32" else x.dtype)
     got = torch.autograd.grad(out, ins, dout)
-    ins = [t.double().requires_grad_(True) for t in leaves]
-    want = torch.autograd.grad(layer64(ins[0], ins[1:4], ins[4]), ins, dout.double())
+    want = layer_grads64(leaves[0], leaves[1:4], leaves[4], dout, EPS)
     for name, a, r in zip(("dx", "dH_pre", "dH_post", "dH_res", "d_w"), got, want):
         assert float((a - r).abs().max() / r.abs().max()) < (TOL[xdt] if name == "dx" else GRAD_TOL), name
 

@@ -10,7 +10,8 @@ import pytest
 import torch
 
 from oracle import mhc_oracle as O
-from tests._helpers import GRAD_TOL, TOL, TORCH_DT, dev_tensor, kernels_missing, np_of, params, rel_err, rng, to_dtype_np
+from tests._helpers import (GRAD_TOL, TOL, TORCH_DT, dev_tensor, kernels_missing, np_of, params, rel_err, rng,
+                            to_dtype_np, tokens_dot)
 
 from mhc_mlx_amd import ops
 from mhc_mlx_amd.reference import mixing_matrix_from_logits
@@ -68,9 +69,8 @@ def test_mxf32_many_slabs_per_wave(T, n, C, knobs):
         ts = [t.clone().requires_grad_(True) for t in (x, M, y)]
         out = ops.stream_mix_add_hip_autograd(*ts)
         res.append([out.detach(), *torch.autograd.grad(out, ts, dout)])
-    ts = [t.double().requires_grad_(True) for t in (x, M, y)]
-    out = torch.matmul(ts[1], ts[0]) + ts[2]
-    res.append([out.detach(), *torch.autograd.grad(out, ts, dout.double())])
+    xd, Md, gd = x.double(), M.double(), dout.double()
+    res.append([torch.matmul(Md, xd) + y.double(), torch.matmul(Md.t().contiguous(), gd), tokens_dot(gd, xd), gd])
     for a, b, r in zip(*res):
         assert float((a - r).abs().max() / r.abs().max()) < 1e-5
         assert float((a - b).abs().max() / r.abs().max()) < 1e-5
@@ -138,7 +138,7 @@ def test_mxf32_dM_is_as_exact_as_the_valu_kernels(T, n, C, knobs):
     """dM at fp32 is no further from float64 than the VALU kernel's (MHC_MIX32=0); see the layer's test of the same name."""
     g = rng(9650 + n)
     x, dout, y = (dev_tensor(g.standard_normal((T, n, C))) for _ in range(3))
-    ref = torch.matmul(dout.double().transpose(0, 1).reshape(n, -1), x.double().transpose(0, 1).reshape(n, -1).t())
+    ref = tokens_dot(dout.double(), x.double())
     err = []
     for on in (1, 0):
         knobs("MHC_MIX32", on)
@@ -162,11 +162,16 @@ def test_mxf32_dispatch_of_large_calls(T, n, C, xdt, odt):
     ins = [t.clone().requires_grad_(True) for t in (x, y, hp, hq, hr)]
     out = ops.post_combine(*ins, sinkhorn_iters=20, eps=1e-5, output_dtype=TORCH_DT[odt])
     got = torch.autograd.grad(out, ins, dout)
-    ins = [t.double().requires_grad_(True) for t in (x, y, hp, hq, hr)]
-    M = mixing_matrix_from_logits(ins[4], iters=20, eps=1e-5) * torch.sigmoid(ins[2])
-    ref = 2 * torch.sigmoid(ins[3]).unsqueeze(-1) * (ins[1] + torch.matmul(M, ins[0]))
-    want = torch.autograd.grad(ref, ins, dout.double())
-    assert float((out.detach() - ref.detach()).abs().max() / ref.detach().abs().max()) < TOL[odt]
+    H = [t.double().requires_grad_(True) for t in (hp, hq, hr)]
+    act = torch.sigmoid(H[0]), 2 * torch.sigmoid(H[1]), mixing_matrix_from_logits(H[2], iters=20, eps=1e-5)
+    a, p, M = (t.detach() for t in act)
+    xd, yd, gd = x.double(), y.double(), dout.double()
+    Mf = p[:, None] * M * a
+    ref = torch.matmul(Mf, xd) + p[:, None] * yd
+    S, Y = tokens_dot(gd, xd), tokens_dot(gd, yd).diagonal()  # sums of g_i x_j and of g_i y_i
+    sums = torch.matmul((S * M).t().contiguous(), p), torch.matmul(S * M, a) + Y, p[:, None] * S * a
+    want = (torch.matmul(Mf.t().contiguous(), gd), p[:, None] * gd, *torch.autograd.grad(act, H, sums))
+    assert float((out.detach() - ref).abs().max() / ref.abs().max()) < TOL[odt]
     for name, a, r in zip(("dx", "dy", "dH_pre", "dH_post", "dH_res"), got, want):
         assert float((a - r).abs().max() / r.abs().max()) < (TOL[xdt] if name in ("dx", "dy") else GRAD_TOL), name
 
