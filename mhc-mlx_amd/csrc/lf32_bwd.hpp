@@ -31,12 +31,13 @@
 // dM, dA and dP are then the wave's own), else up to four.  Above
 // n = 32 (BIG) M^T's operands come from LDS, one 16-row block at a time.
 //
-// Backward kernel, against the VALU kernels before it: 4096 x 32 x 512 fp32
-// 1355 -> 161 us (5.0 TB/s), 4096 x 16 x 1024 fp32 393 -> 140 us (5.8 TB/s),
-// 2048 x 64 x 512 fp32 4145 -> 318 us (one wave per SIMD: dM alone is 64
-// registers), 1024 x 32 x 4096 fp32 3214 -> 400 us, per token 4096 x 32 x 512
-// fp32 1371 -> 190 us and 2500 x 10 x 4000 fp32 479 us (758 us on one wave a token), 3001 x 16 x 1100 fp16 371 -> 101 us and 20000 x 24 x 100
-// bf16 1989 -> 133 us (16-bit rows: bound by the VALU's conversions and LDS).
+// Backward kernel, against the VALU kernels before it, calls replayed over two
+// inputs in turn: 4096 x 32 x 512 fp32 1360 -> 152 us (5.3 TB/s), 4096 x 16 x
+// 1024 fp32 385 -> 141 us (5.7 TB/s), 2048 x 64 x 512 fp32 4138 -> 321 us (one
+// wave per SIMD: dM alone is 64 registers), 1024 x 32 x 4096 fp32 3233 -> 430 us
+// (g read twice), per token 4096 x 32 x 512 fp32 1367 -> 186 us and 2500 x 10 x 4000 fp32 750 -> 369 us, 3001 x 16 x 1100 fp16 346 ->
+// 90 us and 20000 x 24 x 100 bf16 1990 -> 128 us (16-bit rows: bound by the
+// VALU's conversions and LDS).
 #pragma once
 
 #include <type_traits>

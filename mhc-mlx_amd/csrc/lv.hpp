@@ -3,9 +3,9 @@
 // workgroups) do not take, less what tile_fwd_first (fused_fwd.hip) keeps on
 // fused_fwd_kernel, and in the backward two 16-bit operands element by element
 // over more than 2048 channels of more than four streams (one offset per
-// element of both does not fit the registers: bwd_tile_kernel).  At n <= 8 the mix is at most 64 FMAs per channel
-// and HBM is the bound as long as every byte moves once, in wide accesses,
-// with every lane at work, so:
+// element of both does not fit the registers: bwd_tile_kernel).  At n <= 8 the
+// mix is at most 64 FMAs per channel and HBM is the bound as long as every byte
+// moves once, in wide accesses, with every lane at work, so:
 //
 // * A lane holds V channels of all n streams.  Token rows are addressed
 //   through a buffer resource, which takes 16-byte pieces of rows that start

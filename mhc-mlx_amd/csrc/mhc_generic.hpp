@@ -1,4 +1,4 @@
-// Runtime-n kernels for 16 < n <= 64 (generic.hip).
+// Arguments of the kernels with runtime n (generic.hip, lf32_*, lv_*), and the entry points of generic.hip (16 < n <= 64).
 #pragma once
 
 #include <hip/hip_runtime.h>

@@ -14,10 +14,11 @@
 // one's output rows.
 //
 // 8192 x 32 x 32, bf16 x and y, fp32 out and dout, against the VALU kernels
-// before it (one thread per channel, rows of Mf broadcast from LDS): forward
-// 48 -> 20 us (3.4 TB/s), VJP call with its reduction 102 -> 40 us; 8192 x 16 x
-// 128 fp32 39 -> 34 us (6.0 TB/s) and 91 -> 66 us; 8192 x 24 x 40 bf16 36 ->
-// 18 us and 615 -> 39 us; 4096 x 64 x 32 81 -> 24 us and 277 -> 81 us.
+// before it (one thread per channel, rows of Mf broadcast from LDS), calls
+// replayed over two inputs in turn: forward 32 -> 16 us (4.1 TB/s), VJP call
+// with its reduction 96 -> 36 us; 8192 x 16 x 128 fp32 36 -> 33 us (6.1 TB/s)
+// and 87 -> 64 us; 8192 x 24 x 40 bf16 26 -> 16 us and 536 -> 35 us; 4096 x 64 x
+// 32 bf16 60 -> 19 us and 289 -> 76 us.
 #pragma once
 
 #include <type_traits>
