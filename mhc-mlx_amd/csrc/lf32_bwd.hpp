@@ -35,9 +35,9 @@
 // inputs in turn: 4096 x 32 x 512 fp32 1360 -> 152 us (5.3 TB/s), 4096 x 16 x
 // 1024 fp32 385 -> 141 us (5.7 TB/s), 2048 x 64 x 512 fp32 4138 -> 321 us (one
 // wave per SIMD: dM alone is 64 registers), 1024 x 32 x 4096 fp32 3233 -> 430 us
-// (g read twice), per token 4096 x 32 x 512 fp32 1367 -> 186 us and 2500 x 10 x 4000 fp32 750 -> 369 us, 3001 x 16 x 1100 fp16 346 ->
-// 90 us and 20000 x 24 x 100 bf16 1990 -> 128 us (16-bit rows: bound by the
-// VALU's conversions and LDS).
+// (g read twice), per token 4096 x 32 x 512 fp32 1367 -> 186 us and 2500 x 10 x
+// 4000 fp32 750 -> 369 us, 3001 x 16 x 1100 fp16 346 -> 90 us and 20000 x 24 x
+// 100 bf16 1990 -> 128 us (16-bit rows: bound by the VALU's conversions and LDS).
 #pragma once
 
 #include <type_traits>
